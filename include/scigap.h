@@ -119,9 +119,11 @@ int scigap_tv_chambolle(const float* image, float* out,
  * (1..6), continuing from the stored dual field between launches, with the
  * early exit applied after each launch and frames that stopped inside it
  * recomputed.  depth 0: all n_iter_max-1 updates in one launch when they are
- * at most 6, else the autotuned depth (6 when untuned).  Results do not
- * depend on the depth.  The workspace for a given depth is
- * scigap_tv_workspace_bytes_depth(); depth 1 needs the most. */
+ * at most 6, else row sweeps in passes of 3 to 6 updates (or the depth the
+ * autotuner found faster for this shape).  Results do not depend on the
+ * depth.  The workspace for a given depth is
+ * scigap_tv_workspace_bytes_depth(); depth 0 needs the most for more than 6
+ * updates, and runs in chunks of 6 in a workspace sized for another depth. */
 size_t scigap_tv_workspace_bytes_depth(int64_t H, int64_t W, int64_t T, int n_iter_max,
                                        int depth);
 int scigap_tv_chambolle_depth(const float* image, float* out,

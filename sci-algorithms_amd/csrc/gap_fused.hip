@@ -44,6 +44,9 @@ int fill_f64(double* p, int n, double v, hipStream_t s);
 size_t tv_chunked_workspace(int64_t H, int64_t W, int64_t T, int n, int nchunks_max);
 int tv_chunked(const float* image, float* out, int64_t H, int64_t W, int64_t T, float weight,
                float eps, int n, int depth, int* stop_iter, void* ws, hipStream_t s);
+size_t tv_sweep_workspace(int64_t H, int64_t W, int64_t T);
+int tv_sweep(const float* image, float* out, int64_t H, int64_t W, int64_t T, float weight,
+             float eps, int n, int* stop_iter, int* early, void* ws, hipStream_t s);
 int tuned_tv_depth(int64_t H, int64_t W, int64_t T, int n);
 bool tuned_solve_config(const scigap_params& p, int* tile_rows, int* engine);
 
@@ -324,6 +327,12 @@ int max_slot_tiles(int D, int H, int W) {
   return 0;
 }
 
+// Workspace of a deep TV (n - 1 > kMaxFused): row sweeps, or chunks of the
+// depth the autotuner chose for this shape.
+size_t deep_tv_workspace(int64_t H, int64_t W, int64_t T, int n) {
+  return std::max(tv_sweep_workspace(H, W, T), tv_chunked_workspace(H, W, T, n, n - 1));
+}
+
 unsigned grid_pixels(int64_t N) {
   int64_t b = (N + 255) / 256;
   return unsigned(b < 4096 ? (b < 1 ? 1 : b) : 4096);
@@ -363,7 +372,7 @@ Workspace carve(const scigap_params* p, char* base) {
   w.st.nexit = reinterpret_cast<int*>(take(K * 4));
   if (p->tv_iter_max - 1 > kMaxFused) {
     w.vbuf = reinterpret_cast<float*>(take(T * N * 4));
-    w.tvws = take(tv_chunked_workspace(p->H, p->W, p->T, p->tv_iter_max, p->tv_iter_max));
+    w.tvws = take(deep_tv_workspace(p->H, p->W, p->T, p->tv_iter_max));
   }
   w.bytes = off;
   return w;
@@ -541,11 +550,16 @@ int scigap_solve(const scigap_params* p, const float* y, const float* phi, const
       pa.x_out = ws.vbuf;
       k_gap_proj<<<grid_pixels(N), 256, 0, s>>>(pa);
       SCIGAP_LAUNCH_CHECK("projection launch");
-      if (int rc = tv_chunked(ws.vbuf, a.x_out, p->H, p->W, T, a.weight, p->tv_eps,
-                              p->tv_iter_max, deep_depth, stats ? ws.st.stop : nullptr,
-                              ws.tvws, s))
+      if (deep_depth == 0) {
+        if (int rc = tv_sweep(ws.vbuf, a.x_out, p->H, p->W, T, a.weight, p->tv_eps,
+                              p->tv_iter_max, nullptr, stats ? stats + k : nullptr, ws.tvws, s))
+          return rc;
+      } else if (int rc = tv_chunked(ws.vbuf, a.x_out, p->H, p->W, T, a.weight, p->tv_eps,
+                                     p->tv_iter_max, deep_depth, stats ? ws.st.stop : nullptr,
+                                     ws.tvws, s)) {
         return rc;
-      if (stats) {  // frames whose TV stopped early in this iteration
+      }
+      if (stats && deep_depth) {  // frames whose TV stopped early in this iteration
         k_count_early<<<1, 256, 0, s>>>(ws.st.stop, int(T), p->tv_iter_max - 1, stats + k);
         SCIGAP_LAUNCH_CHECK("early-stop count launch");
       }
@@ -580,7 +594,8 @@ size_t scigap_tv_workspace_bytes_depth(int64_t H, int64_t W, int64_t T, int n_it
   if (depth >= D)
     return align256(size_t(T) * D * size_t(max_slot_tiles(D, int(H), int(W))) * 4) +
            align256(size_t(T) * 4) + 256;
-  return tv_chunked_workspace(H, W, T, n_iter_max, D);
+  return depth == 0 ? deep_tv_workspace(H, W, T, n_iter_max)
+                    : tv_chunked_workspace(H, W, T, n_iter_max, D);
 }
 
 size_t scigap_tv_workspace_bytes(int64_t H, int64_t W, int64_t T, int n_iter_max) {
@@ -602,7 +617,14 @@ int scigap_tv_chambolle_depth(const float* image, float* out, int64_t H, int64_t
     return fail(SCIGAP_EINVAL, "H*W must be <= 2^30 - 8 (buffer-addressed planes)");
   const size_t vol = size_t(H * W * T) * 4;
   if (overlaps(image, vol, out, vol)) return fail(SCIGAP_EALIAS, "image and out overlap");
-  const size_t need = scigap_tv_workspace_bytes_depth(H, W, T, n_iter_max, depth);
+  size_t need = scigap_tv_workspace_bytes_depth(H, W, T, n_iter_max, depth);
+  // A workspace sized for an explicit depth does for depth 0 as well: the
+  // chunks run in it then.
+  bool sweep_fits = true;
+  if (depth == 0 && n_iter_max - 1 > kMaxFused && workspace_bytes < need) {
+    need = tv_chunked_workspace(H, W, T, n_iter_max, n_iter_max - 1);
+    sweep_fits = false;
+  }
   if (!workspace || workspace_bytes < need)
     return fail(SCIGAP_EWORKSPACE, "workspace needs %zu bytes, got %zu", need, workspace_bytes);
   if ((reinterpret_cast<uintptr_t>(image) | reinterpret_cast<uintptr_t>(out)) % 8 != 0)
@@ -620,6 +642,10 @@ int scigap_tv_chambolle_depth(const float* image, float* out, int64_t H, int64_t
     return SCIGAP_OK;
   }
   if (depth == 0) depth = D <= kMaxFused ? D : tuned_tv_depth(H, W, T, n_iter_max);
+  if (depth == 0 && !sweep_fits) depth = kMaxFused;
+  if (depth == 0)
+    return tv_sweep(image, out, H, W, T, weight, eps, n_iter_max, stop_iter, nullptr, workspace,
+                    s);
   if (depth < D)
     return tv_chunked(image, out, H, W, T, weight, eps, n_iter_max, depth, stop_iter, workspace,
                       s);

@@ -7,7 +7,8 @@
 // variable SCIGAP_TUNE_CACHE names a file, entries are loaded from it on
 // first use and every new entry is appended to it, so later processes start
 // tuned.  scigap_solve uses a cached entry when its tile_rows and engine are
-// both 0; scigap_tv_chambolle uses the cached depth for depth 0.
+// both 0; scigap_tv_chambolle uses the cached depth for depth 0 (an entry of
+// depth 0 says that the row sweeps beat every depth).
 
 #include <hip/hip_runtime.h>
 
@@ -81,6 +82,12 @@ void store(const Key& k, const Entry& e) {
   }
 }
 
+void forget(const Key& k) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  load_locked();
+  g_cache.erase(k);
+}
+
 bool lookup(const Key& k, Entry* e) {
   std::lock_guard<std::mutex> lock(g_mu);
   load_locked();
@@ -129,12 +136,13 @@ double time_on_stream(F&& fn, hipStream_t s, int reps, int* rc) {
 
 }  // namespace
 
-// Tuned TV fusion depth for a deep TV (n - 1 > 6 updates); 6 when untuned.
+// Tuned TV fusion depth for a deep TV (n - 1 > 6 updates); 0 (row sweeps,
+// tv_sweep.hip) when untuned or when the sweeps were the fastest.
 int tuned_tv_depth(int64_t H, int64_t W, int64_t T, int n) {
   Entry e;
   if (lookup(Key(1, H, W, T, 0, n), &e) && e.depth >= 1 && e.depth <= max_chunk_depth())
     return e.depth;
-  return max_chunk_depth();
+  return 0;
 }
 
 // Tuned (tile_rows, engine) of a solve shape, if any.
@@ -215,6 +223,21 @@ int scigap_autotune_tv(const float* image, float* out, int64_t H, int64_t W, int
   double def_ms = -1.0;
   int n = 0;
   const int dmax = max_chunk_depth();
+  // The untuned path (depth 0) is not a candidate, but a depth is remembered
+  // only if it beats it.
+  const Key key(1, H, W, T, 0, n_iter_max);
+  forget(key);
+  double untuned_ms = -1.0;
+  if (D > dmax && workspace_bytes >= scigap_tv_workspace_bytes_depth(H, W, T, n_iter_max, 0)) {
+    int rc = SCIGAP_OK;
+    untuned_ms = time_on_stream(
+        [&]() {
+          return scigap_tv_chambolle_depth(image, out, H, W, T, weight, eps, n_iter_max, 0,
+                                           nullptr, workspace, workspace_bytes, stream);
+        },
+        s, 2, &rc);
+    if (rc != SCIGAP_OK) return rc;
+  }
   for (int d = dmax; d >= 1; --d) {
     if (d > D) continue;
     int rc = SCIGAP_OK;
@@ -232,7 +255,12 @@ int scigap_autotune_tv(const float* image, float* out, int64_t H, int64_t W, int
       best.ms = ms;
     }
   }
-  store(Key(1, H, W, T, 0, n_iter_max), best);
+  Entry keep = best;
+  if (untuned_ms >= 0.0 && untuned_ms <= best.ms) {
+    keep.depth = 0;
+    keep.ms = untuned_ms;
+  }
+  store(key, keep);
   res->tile_rows = 0;
   res->engine = 0;
   res->tv_depth = best.depth;

@@ -1,4 +1,5 @@
-// Chambolle TV of any depth in chunks of up to 6 fused dual updates.
+// Chambolle TV of any depth in chunks of an explicit number (1..6) of fused
+// dual updates (the default deep TV is tv_sweep.hip).
 //
 // scikit-image's denoise_tv_chambolle (0.18.3 restoration/_denoise.py:341-393)
 // runs n_iter_max - 1 dual updates per frame; the legacy solvers use 30

@@ -57,7 +57,7 @@ def autotune_tv(image_thw, *, weight=0.1, eps=2e-4, n_iter_max=30):
     import torch
     L = _lib.lib()
     T, H, W = image_thw.shape
-    nbytes = L.scigap_tv_workspace_bytes_depth(H, W, T, int(n_iter_max), 1)
+    nbytes = max(L.scigap_tv_workspace_bytes_depth(H, W, T, int(n_iter_max), d) for d in (0, 1))
     ws = torch.empty(nbytes, dtype=torch.uint8, device=image_thw.device)
     out = torch.empty_like(image_thw)
     r = _lib.TuneResult()

@@ -1,0 +1,37 @@
+"""Row-sweep kernels on the device against the FP64 oracle, at the sizes where
+strips, blocks of rows and passes begin and end."""
+
+import numpy as np
+import pytest
+
+import pnp_sci_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _frames(H, W, T, seed):
+    """Frames that stop at different depths: a smooth image under growing noise."""
+    g = np.random.default_rng(seed)
+    r, c = np.arange(H)[:, None], np.arange(W)[None]
+    base = 0.5 + 0.3 * np.cos(2 * np.pi * (r / 50 + c / 70))
+    return np.stack([base + (0.02 + 0.1 * t) * g.standard_normal((H, W)) for t in range(T)])
+
+
+@pytest.mark.parametrize("n", [8, 13, 14, 30])       # passes 4+3, 6+6, 5+4+4, 6+6+6+6+5
+@pytest.mark.parametrize("H,W", [(1, 300), (300, 1), (7, 9), (8, 127), (9, 128), (63, 129),
+                                 (64, 232), (65, 243), (130, 518)])
+def test_deep_tv_passes_match_oracle(gpu, H, W, n):
+    """The default deep TV: image and exit iteration of every frame, for frames
+    that stop inside the first, a middle and the last pass and for ones that
+    run to the end (max abs error 2e-5, the bound of the TV tests)."""
+    import torch
+    from pnp_sci.tv import tv_device
+    img = _frames(H, W, 3, 1000 * H + W).astype(np.float32)
+    for eps in (2e-4, 1e-2):
+        got, stop = tv_device(torch.tensor(img, device="cuda"), 0.1, eps, n, return_stop=True)
+        got, stop = got.cpu().numpy(), stop.cpu().tolist()
+        for t in range(img.shape[0]):
+            st = {}
+            want = O.tv_chambolle_nd(img[t].astype(np.float64), 0.1, eps, n, _stats=st)
+            assert stop[t] == st["returned"], (eps, t)
+            assert np.max(np.abs(got[t] - want)) <= 2e-5, (eps, t)
