@@ -1,5 +1,7 @@
 // Fused reverse pass of the fixed-depth Chambolle TV used by the unrolled
-// GAP-TV (one workgroup per tile and frame).
+// GAP-TV: row sweeps for D <= 4 (second half of this file), one workgroup per
+// tile and frame for D = 5, 6, whose states in waiting (2r rows of forward
+// update D-1-r) would need more registers than a wave has.
 //
 // Forward (D updates from p_0 = 0, c = tau/w, tau = 1/4; G the masked
 // forward difference, G^T its transpose, scikit-image 0.18.3
@@ -27,9 +29,14 @@
 // 128-4D x 64-4D interior, and up to the image edge on a side where the tile
 // meets it (nothing is stale there: the masks are exact).
 
-#include "fused.h"
+#include "sweep.h"
+
+#include <algorithm>
+#include <cmath>
 
 namespace scigap {
+
+int device_simds();
 
 namespace {
 
@@ -379,6 +386,281 @@ int launch_tv_bwd(BwdArgs a, int T, hipStream_t s) {
   return SCIGAP_OK;
 }
 
+// ---------------------------------------------------------------------------
+// The same reverse as a row sweep (D <= 4): one wave per strip and frame, no
+// recomputation and no LDS.
+// ---------------------------------------------------------------------------
+//
+// Row i of v arrives at step i; forward update u is at row i - 1 - u, and
+// reverse step u = D-1-r, which needs g_u, p_u of its row and rows of
+// pbar_{u+1}, is at row i - D - r: 2r rows behind the forward update whose
+// state it takes, which waits for it in registers (rings over the row number).
+// The reverse runs in Z = -tau pbar and q = -4p = b s with b = q_u + g:
+//   A = Z s,  t = <Z, b>,  gbar = A - c s^2 t g/n,  obar = G^T gbar,
+//   vbar += obar,  Z_u = A - tau G obar,  cbar -= n s^2 t,
+// the formulas above with every tau a power of two.  2D-1 halo rows and 2D
+// halo columns on a side that is not the image edge.
+//
+// What bounds it: vector instruction issue (about 330 a row of 128 columns for
+// D = 4, 32 of them square roots and reciprocals), at two waves a SIMD (256
+// registers for D = 4).  Alone at 1024x1024x20, D = 4: 145-190 us against
+// 620 us of the tile kernel above; 18 against 27 us at 256x256x8.
+
+constexpr int kBwdAhead = 2;  // rows requested ahead of their use
+constexpr int kBwdWaves = 4;  // independent waves of one workgroup
+
+struct BwdSweepArgs {
+  BwdArgs b;
+  int T, R, strips_x, strips, items, per_xcd;
+};
+
+using namespace sweep;
+
+// Masked forward difference of rows a (j) and b (j+1): g0 vertical, g1
+// horizontal, as dual_step forms it.
+template <bool EDGE>
+__device__ __forceinline__ void diff_row(f2 a, f2 b, const StripPos& sp, bool vrow, f2& g0,
+                                         f2& g1) {
+  const float right1 = from_next_lane(a.x);
+  g0 = f2{b.x - a.x, b.y - a.y};
+  g1 = f2{a.y - a.x, right1 - a.y};
+  if constexpr (EDGE) {
+    g0.x = vrow ? g0.x : 0.f;
+    g0.y = vrow ? g0.y : 0.f;
+    g1.x = sp.h0 ? g1.x : 0.f;
+    g1.y = sp.h1 ? g1.y : 0.f;
+  }
+}
+
+// G^T of a row: a0 (with the row above's in `up`) and a1.
+__device__ __forceinline__ f2 adj_row(f2 a0, f2 a1, f2 up) {
+  const float left0 = from_prev_lane(a1.y);
+  return f2{(up.x - a0.x) + (left0 - a1.x), (up.y - a0.y) + (a1.x - a1.y)};
+}
+
+template <int D, bool EDGE>
+struct BwdRows {
+  static constexpr int kHalo = 2 * D - 1;
+  static constexpr int kFill = 4 * D - 2;  // steps before the first finished row
+  f2 v[kRing], xb[kRing];                  // v; xbar, then vbar as it accumulates
+  f2 out[D][kRing];                        // out_u
+  f2 q0[D + 1][kRing], q1[D + 1][kRing];   // q_u
+  f2 g0[D][kRing], g1[D][kRing];           // g_u
+  f2 n[D][kRing];                          // |g_u|
+  f2 z0[D + 1][kRing], z1[D + 1][kRing];   // Z_u
+  f2 A0[D][kRing], A1[D][kRing];           // A of reverse step u
+  f2 gb0[D][kRing];                        // gbar (vertical) of reverse step u
+  f2 ob[D][kRing];                         // obar of reverse step u
+  double cb = 0.0;                         // sum of -n s^2 t over owned pixels
+
+  // Step I (v of row I and xbar of row I - D + 1 already stored); `row` is
+  // row I's global row.  FILL, M, `last` as in Rows::step.
+  template <int I, bool FILL>
+  __device__ __forceinline__ void step(const StripPos& sp, int row, int H, float tw, bool last) {
+    constexpr int M = FILL ? 0 : (I - kFill);
+    constexpr int B = kRing * 8;
+    auto vrow = [&](int r) { return !EDGE || (r >= 0 && r < H - 1); };
+    out[0][I % kRing] = v[I % kRing];
+    // Forward updates: g_u, |g_u|, q_{u+1}, out_{u+1} of row I - 1 - u.
+    static_for<D>([&](auto uc) __attribute__((always_inline)) {
+      constexpr int u = decltype(uc)::value;
+      if constexpr (!FILL || I >= 2 * u + 1) {
+        constexpr int j = (I + B - 1 - u) % kRing, jn = (j + 1) % kRing, jp = (j + kRing - 1) % kRing;
+        diff_row<EDGE>(out[u][j], out[u][jn], sp, vrow(row - 1 - u), g0[u][j], g1[u][j]);
+        const f2 a = g0[u][j], b = g1[u][j];
+        const float n0 = fast_sqrt(fmaf(a.x, a.x, b.x * b.x));
+        const float n1 = fast_sqrt(fmaf(a.y, a.y, b.y * b.y));
+        n[u][j] = f2{n0, n1};
+        if constexpr (u + 1 < D) {
+          const float s0 = fast_rcp(fmaf(tw, n0, 1.f)), s1 = fast_rcp(fmaf(tw, n1, 1.f));
+          const f2 c = u ? f2{q0[u][j].x + a.x, q0[u][j].y + a.y} : a;
+          const f2 d = u ? f2{q1[u][j].x + b.x, q1[u][j].y + b.y} : b;
+          q0[u + 1][j] = f2{c.x * s0, c.y * s1};
+          q1[u + 1][j] = f2{d.x * s0, d.y * s1};
+          if constexpr (!FILL || I >= 2 * u + 2) {
+            const f2 o = adj_row(q0[u + 1][j], q1[u + 1][j], q0[u + 1][jp]);
+            out[u + 1][j] = f2{fmaf(-0.25f, o.x, v[j].x), fmaf(-0.25f, o.y, v[j].y)};
+          }
+        }
+      }
+    });
+    // Z_D of row I - D.
+    if constexpr (!FILL || I >= 2 * D - 1) {
+      constexpr int j = (I + B - D) % kRing, jn = (j + 1) % kRing;
+      f2 a, b;
+      diff_row<EDGE>(xb[j], xb[jn], sp, vrow(row - D), a, b);
+      z0[D][j] = f2{-0.25f * a.x, -0.25f * a.y};
+      z1[D][j] = f2{-0.25f * b.x, -0.25f * b.y};
+    }
+    // Reverse step u = D-1-r at row I - D - r, then Z_u of the row above.
+    float c = 0.f;
+    static_for<D>([&](auto rc) __attribute__((always_inline)) {
+      constexpr int r = decltype(rc)::value, u = D - 1 - r;
+      if constexpr (!FILL || I >= 2 * D - 1 + 2 * r) {
+        constexpr int j = (I + B - D - r) % kRing, jp = (j + kRing - 1) % kRing;
+        const f2 a = g0[u][j], b = g1[u][j], Z0 = z0[u + 1][j], Z1 = z1[u + 1][j];
+        f2 G0, G1;
+        float ct = 0.f;
+        static_for<2>([&](auto kc) __attribute__((always_inline)) {
+          constexpr int k = decltype(kc)::value;
+          const float nn = n[u][j][k];
+          const float s = fast_rcp(fmaf(tw, nn, 1.f));
+          const float b0 = u ? q0[u][j][k] + a[k] : a[k], b1 = u ? q1[u][j][k] + b[k] : b[k];
+          const float a0 = Z0[k] * s, a1 = Z1[k] * s;
+          const float t = fmaf(Z0[k], b0, Z1[k] * b1);
+          const float w = s * s * t;
+          // -c s^2 t / n (hardware reciprocal, about 1 ulp; 0 where n = 0)
+          const float kk = nn > 0.f ? -tw * w * fast_rcp(nn) : 0.f;
+          A0[u][j][k] = a0;
+          A1[u][j][k] = a1;
+          G0[k] = fmaf(kk, a[k], a0);
+          G1[k] = fmaf(kk, b[k], a1);
+          ct = (k == 0 ? sp.owner : sp.own1 && sp.owner) ? fmaf(-nn, w, ct) : ct;
+        });
+        // Row I - D - r adds to the weight's adjoint when the strip owns it:
+        // rows [kHalo, kHalo + R), with I - D - r the strip's row.
+        if constexpr (!FILL || I - D - r >= kHalo) {
+          constexpr bool cut = !FILL && (M + 2 * D - 1 - D - r >= kRing);
+          c += cut && last ? 0.f : ct;
+        }
+        gb0[u][j] = G0;
+        if constexpr (!FILL || I >= 2 * D + 2 * r) {
+          const f2 o = adj_row(G0, G1, gb0[u][jp]);
+          ob[u][j] = o;
+          xb[j] = f2{xb[j].x + o.x, xb[j].y + o.y};
+        }
+        if constexpr (u > 0 && (!FILL || I >= 2 * D + 2 * r + 1)) {
+          f2 da, db;
+          diff_row<EDGE>(ob[u][jp], ob[u][j], sp, vrow(row - D - r - 1), da, db);
+          z0[u][jp] = f2{fmaf(-0.25f, da.x, A0[u][jp].x), fmaf(-0.25f, da.y, A0[u][jp].y)};
+          z1[u][jp] = f2{fmaf(-0.25f, db.x, A1[u][jp].x), fmaf(-0.25f, db.y, A1[u][jp].y)};
+        }
+      }
+    });
+    cb += double(c);
+    asm volatile("" : "+v"(cb));
+  }
+};
+
+template <int D, bool EDGE>
+__device__ __forceinline__ double bwd_strip(const BwdSweepArgs& s, const Strip& st, int t) {
+  using E = BwdRows<D, EDGE>;
+  constexpr int P = kBwdAhead, FILL = E::kFill, HALO = E::kHalo;
+  const BwdArgs& a = s.b;
+  const int H = a.H, W = a.W, N = H * W;
+  const StripPos& sp = st.sp;
+  const int vo = (sp.row0 * W + sp.col) * 4;
+  const unsigned vst = sp.owner ? unsigned(vo) : kNoStore;
+  const __amdgpu_buffer_rsrc_t rr = plane_rsrc(a.r, N);
+  const __amdgpu_buffer_rsrc_t rx = plane_rsrc(a.x + size_t(t) * N, N);
+  const __amdgpu_buffer_rsrc_t rf = plane_rsrc(a.phi + size_t(t) * N, N);
+  const __amdgpu_buffer_rsrc_t rb = plane_rsrc(a.xbar + size_t(t) * N, N);
+  // No ybb: zero records read as 0.
+  const __amdgpu_buffer_rsrc_t ry = plane_rsrc(a.ybb, a.ybb ? N : 0);
+  const __amdgpu_buffer_rsrc_t wv = plane_rsrc(a.vbar + size_t(t) * N, N);
+  E e;
+  f2 nx[P], nf[P], nb[P];
+  f2 nr, ny, ng;  // read before or by other frames as well (Phi of xbar's row): one row ahead
+  const float tw = a.tw, lam = a.lam;
+  const int rows_all = s.R + 2 * HALO;
+  // Requests of step i: v's row i and xbar's row i - D + 1.
+  auto request = [&](auto pc, int i) __attribute__((always_inline)) {
+    constexpr int p = decltype(pc)::value % P;
+    const int k = i < rows_all ? i : rows_all - 1;  // past the end: the last row again
+    const int kb = k - D + 1 > 0 ? k - D + 1 : 0;
+    nf[p] = load_px<EDGE>(rf, sp, vo, k, H, W);
+    nx[p] = load_px<EDGE>(rx, sp, vo, k, H, W);
+    nb[p] = load_px<EDGE>(rb, sp, vo, kb, H, W);
+  };
+  auto request_planes = [&](int i) __attribute__((always_inline)) {
+    const int k = i < rows_all ? i : rows_all - 1;
+    nr = load_px<EDGE>(rr, sp, vo, k, H, W);
+    const int kb = k - D + 1 > 0 ? k - D + 1 : 0;
+    ny = load_px<EDGE>(ry, sp, vo, kb, H, W);
+    ng = load_px<EDGE>(rf, sp, vo, kb, H, W);
+  };
+  request_planes(0);
+  static_for<P>([&](auto k) __attribute__((always_inline)) { request(k, decltype(k)::value); });
+  auto feed = [&](auto ic, int i) __attribute__((always_inline)) {
+    constexpr int I = decltype(ic)::value, sl = I % kRing, p = I % P;
+    constexpr int xl = (I + kRing * 8 - D + 1) % kRing;
+    e.v[sl] = f2{fmaf(nr.x * lam, nf[p].x, nx[p].x), fmaf(nr.y * lam, nf[p].y, nx[p].y)};
+    e.xb[xl] = f2{fmaf(ny.x, ng.x, nb[p].x), fmaf(ny.y, ng.y, nb[p].y)};
+    request_planes(i + 1);
+    request(std::integral_constant<int, p>{}, i + P);
+  };
+  static_for<FILL>([&](auto ic) __attribute__((always_inline)) {
+    constexpr int i = decltype(ic)::value;
+    feed(ic, i);
+    e.template step<i, true>(sp, sp.row0 + i, H, tw, false);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+#pragma unroll 1
+  for (int b = 0; b < s.R; b += kRing) {
+    const bool last = b + kRing >= s.R;
+    static_for<kRing>([&](auto mc) __attribute__((always_inline)) {
+      constexpr int m = decltype(mc)::value, I = FILL + m;
+      constexpr int j = (I + kRing * 8 - HALO) % kRing;  // slot of the finished row
+      const int i = FILL + b + m;
+      feed(std::integral_constant<int, I>{}, i);
+      e.template step<I, false>(sp, sp.row0 + i, H, tw, last);
+      store_px<EDGE>(wv, sp, vst, i - HALO, H, W, e.xb[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+  return e.cb;
+}
+
+template <int D>
+__global__ void __launch_bounds__(64 * kBwdWaves) __attribute__((amdgpu_waves_per_eu(2)))
+k_tv_bwd_sweep(BwdSweepArgs s) {
+  __shared__ double red[kBwdWaves];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int item = tile_of_block(blockIdx.x, s.per_xcd) * kBwdWaves + w;
+  double cb = 0.0;
+  if (item < s.items) {
+    const int t = item / s.strips, strip = item - t * s.strips;
+    constexpr int HALO = 2 * D - 1;
+    const Strip st(strip, s.strips_x, s.b.H, s.b.W, s.R, 2 * D, HALO, HALO);
+    cb = st.edge ? bwd_strip<D, true>(s, st, t) : bwd_strip<D, false>(s, st, t);
+  }
+  // Weight adjoint: one double atomic per workgroup.
+  cb = wave_sum(cb);
+  if ((threadIdx.x & 63) == 0) red[w] = cb;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double tot = 0.0;
+    for (int k = 0; k < kBwdWaves; ++k) tot += red[k];
+    if (tot != 0.0) atomicAdd(s.b.wbar, tot * s.b.wscale);
+  }
+}
+
+// Rows a strip owns (see tv_sweep.hip): a strip of R rows costs about
+// R + 10 full rows, and a SIMD is about 2/3 busy with a single wave.
+template <int D>
+int launch_tv_bwd_sweep(const BwdArgs& a, int T, hipStream_t s) {
+  BwdSweepArgs g{};
+  g.b = a;
+  g.T = T;
+  g.strips_x = tiles_across(a.W, 128, 2 * D, 128 - 4 * D);
+  const double simds = device_simds();
+  double best = 1e300;
+  for (int R : {8, 16, 32, 64}) {
+    const double waves = double(g.strips_x) * ((a.H + R - 1) / R) * T;
+    const double cost = std::max(1.5, std::ceil(waves / simds)) * (R + 10);
+    if (cost < best * 0.999) {
+      best = cost;
+      g.R = R;
+    }
+  }
+  g.strips = g.strips_x * ((a.H + g.R - 1) / g.R);
+  g.items = g.strips * T;
+  g.per_xcd = ((g.items + kBwdWaves - 1) / kBwdWaves + 7) / 8;
+  k_tv_bwd_sweep<D><<<unsigned(g.per_xcd * 8), 64 * kBwdWaves, 0, s>>>(g);
+  SCIGAP_LAUNCH_CHECK("TV backward sweep launch");
+  return SCIGAP_OK;
+}
+
 }  // namespace
 
 // vbar = (d out_D / d v)^T xbar for every frame, and wbar += xbar . d out_D / dw,
@@ -401,10 +683,10 @@ int tv_backward_tiles(int D, const float* x, const float* phi, const float* r, f
   a.tw = float(0.25 / double(w));
   a.wscale = -double(kTauB) / (double(w) * double(w));
   switch (D) {
-    case 1: return launch_tv_bwd<1>(a, int(T), s);
-    case 2: return launch_tv_bwd<2>(a, int(T), s);
-    case 3: return launch_tv_bwd<3>(a, int(T), s);
-    case 4: return launch_tv_bwd<4>(a, int(T), s);
+    case 1: return launch_tv_bwd_sweep<1>(a, int(T), s);
+    case 2: return launch_tv_bwd_sweep<2>(a, int(T), s);
+    case 3: return launch_tv_bwd_sweep<3>(a, int(T), s);
+    case 4: return launch_tv_bwd_sweep<4>(a, int(T), s);
     case 5: return launch_tv_bwd<5>(a, int(T), s);
     case 6: return launch_tv_bwd<6>(a, int(T), s);
   }

@@ -35,3 +35,21 @@ def test_deep_tv_passes_match_oracle(gpu, H, W, n):
             want = O.tv_chambolle_nd(img[t].astype(np.float64), 0.1, eps, n, _stats=st)
             assert stop[t] == st["returned"], (eps, t)
             assert np.max(np.abs(got[t] - want)) <= 2e-5, (eps, t)
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5])          # 1..4 dual updates
+@pytest.mark.parametrize("H,W", [(1, 130), (7, 113), (8, 112), (9, 128), (16, 127), (33, 226),
+                                 (65, 240)])
+def test_reverse_sweep_matches_fp64_autograd(gpu, H, W, n):
+    """The reverse TV at the edges of strips and blocks of rows: gradients of
+    the mask, lambda and weights against FP64 autograd (the bounds of the
+    unrolled tests: 1e-4 forward, 1e-3 gradients)."""
+    from pnp_sci.synthetic import unrolled_batch
+    from test_gpu_unrolled import _hip, _ref, _schedules, rel
+    truth, mask = unrolled_batch(1, H, W, 3, seed=H * W, mask="logits")
+    lam, w = _schedules(2, n)
+    got = _hip(mask, truth, lam, w, n, True)
+    want = _ref(mask, truth, lam, w, n, True)
+    assert rel(got["x"], want["x"]) <= 1e-4
+    for k in ("mask", "lam", "w"):
+        assert rel(got[k], want[k]) <= 1e-3, k
