@@ -339,9 +339,10 @@ __device__ __forceinline__ void store_owned(float* __restrict__ p, int N, int W,
 // One tile of one fused outer iteration (the body of k_fused and of the
 // batched persistent kernel).  Returns without work when the tile's class
 // (interior/border) differs from INSIDE.  X1 selects the one-barrier TV
-// engine (tv_run_x1).
+// engine (tv_run_x1).  ENERGY false: no exit test follows and no energies are
+// formed.
 template <int D, int BY, int MR, int MODE, bool INSIDE, bool IQA, bool X1 = false,
-          bool DMA = false>
+          bool DMA = false, bool ENERGY = true>
 __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
                                            FusedLds<D, BY, MR, X1, DMA>& sh, int part = 0) {
   using G = TileGeom<D, BY, MR>;
@@ -412,8 +413,9 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
       }
     }
   }
-  for (int i = threadIdx.x; i < kEnergyFrames * BY * EnergySlots<D>::kPerWave; i += blockDim.x)
-    red[i] = 0.f;
+  if constexpr (ENERGY)
+    for (int i = threadIdx.x; i < kEnergyFrames * BY * EnergySlots<D>::kPerWave; i += blockDim.x)
+      red[i] = 0.f;
   float err = 0.f;
 
   // Frame t+1's x and Phi are requested before frame t's TV so that their
@@ -514,11 +516,11 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
     float out[RY][2];
     float acc[NH * 8];
     if constexpr (X1) {
-      tv_run_x1<D, RY, BY, NH, !INSIDE>(img, out, D, lds, lp, em, a.weight, a.tw, acc, true,
+      tv_run_x1<D, RY, BY, NH, !INSIDE>(img, out, D, lds, lp, em, a.weight, a.tw, acc, ENERGY,
                                         prefetch);
     } else
       tv_run_from_zero<D, RY, BY, NH, !INSIDE>(img, out, D, lds, lp, em, a.weight, a.tw, acc,
-                                               true, prefetch);
+                                               ENERGY, prefetch);
 
     if (owns_any) {
       float bv[RY][2];
@@ -582,10 +584,12 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
           }
       }
     }
-    const int tb = t % kEnergyFrames;
-    energy_add<D, BY, MR, NH>(acc, tp.lane_owner, red + tb * BY * EnergySlots<D>::kPerWave, lp);
-    if (es && (tb == kEnergyFrames - 1 || t == T - 1))  // workgroup-uniform
-      energy_store<D, BY>(red, tb + 1, es - size_t(tb) * D * es_stride, es_stride, tile_id);
+    if constexpr (ENERGY) {
+      const int tb = t % kEnergyFrames;
+      energy_add<D, BY, MR, NH>(acc, tp.lane_owner, red + tb * BY * EnergySlots<D>::kPerWave, lp);
+      if (es && (tb == kEnergyFrames - 1 || t == T - 1))  // workgroup-uniform
+        energy_store<D, BY>(red, tb + 1, es - size_t(tb) * D * es_stride, es_stride, tile_id);
+    }
     phit += N;
     xt += N;
     xo += N;

@@ -29,11 +29,8 @@
 // and Phi as the forward did and recomputes the inner dual fields in
 // registers.  Layout (T,H,W) per sample.
 
-#include <algorithm>
 #include <cmath>
-#include <map>
-#include <mutex>
-#include <vector>
+#include <initializer_list>
 
 #include "scigap_internal.h"
 
@@ -41,21 +38,44 @@ namespace scigap {
 
 namespace {
 
-constexpr int BX = 64, BYR = 4;  // 256-thread blocks of the per-pixel kernels
-constexpr int kGroup = 4;        // frames whose loads a per-pixel kernel issues together
-constexpr float kTau = 0.25f;
+constexpr int kThreads = 256;
+constexpr int kSamples = 4;  // samples of one launch (a group)
 
-// Block reduction of one float into a double accumulator (scaled).
-__device__ __forceinline__ void block_atomic(float v, double* dst, double scale) {
+// Block reduction of one float into a gradient accumulator's slot.
+__device__ __forceinline__ void block_atomic(float v, double* dst) {
   const float s = wave_sum(v);
-  __shared__ float part[BX * BYR / 64];
+  __shared__ float part[kThreads / 64];
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) {
     double tot = 0.0;
-    for (int w = 0; w < BX * BYR / 64; ++w) tot += part[w];
-    atomicAdd(dst, tot * scale);
+    for (int w = 0; w < kThreads / 64; ++w) tot += part[w];
+    atomicAdd(grad_slot(dst), tot);
   }
+}
+
+// V consecutive floats of a plane.
+template <int V>
+struct Vec {
+  float v[V];
+};
+template <int V>
+__device__ __forceinline__ Vec<V> ldv(const float* p, int64_t i) {
+  Vec<V> r;
+  if constexpr (V == 4) {
+    const float4 f = reinterpret_cast<const float4*>(p)[i];
+    r.v[0] = f.x, r.v[1] = f.y, r.v[2] = f.z, r.v[3] = f.w;
+  } else {
+    r.v[0] = p[i];
+  }
+  return r;
+}
+template <int V>
+__device__ __forceinline__ void stv(float* p, int64_t i, const Vec<V>& r) {
+  if constexpr (V == 4)
+    reinterpret_cast<float4*>(p)[i] = make_float4(r.v[0], r.v[1], r.v[2], r.v[3]);
+  else
+    p[i] = r.v[0];
 }
 
 // Reverse of the projection v = x + lambda*r*Phi, r = (y1' - yb)/S,
@@ -65,102 +85,183 @@ __device__ __forceinline__ void block_atomic(float v, double* dst, double scale)
 // ybar += y1bar', Sbar = -rbar r / S.  The frame part xbar_t = vbar_t + ybb Phi_t
 // is never stored: the next reverse TV step forms it on load, and the mask
 // gradient (k_ub_phibar) takes ybb and Sbar from the planes written here.
-__global__ void __launch_bounds__(256) k_ub_proj(
-    const float* __restrict__ vbar, const float* __restrict__ phi, const float* __restrict__ S,
-    const float* __restrict__ r, float lam, const float* __restrict__ y1bar_ext,
-    float* __restrict__ y1bar_out, float* __restrict__ ybar, float* __restrict__ ybb_out,
-    float* __restrict__ sbar_out, double* lambar, int64_t N, int T) {
+// blockIdx.y is the sample; planes of N, volumes of N*T floats per sample, r
+// at its own distance.
+//
+// Memory-bound: V = 4 (16 bytes a lane) where that leaves waves enough; the
+// loads of G frames are issued together (one memory latency per group), the
+// sums keep frame order.  2 x 1024x1024x20: 58 us, against 78 us for each of two
+// concurrent launches of one sample with one pixel a lane; 4 x 256x256x8: 6.5 us.
+struct ProjArgs {
+  const float* vbar;
+  const float* phi;
+  const float* S;
+  const float* r;
+  size_t r_b;
+  float lam;
+  const float* y1bar_in;  // null: 0
+  float* y1bar_out;
+  float* ybar;
+  float* ybb;
+  float* sbar;  // null: no mask gradient
+  double* lambar;
+  int64_t N;
+  int T;
+};
+
+template <int V, int G>
+__global__ void __launch_bounds__(kThreads) k_ub_proj(ProjArgs a) {
+  const int b = blockIdx.y;
+  const int64_t n = a.N / V;
+  const size_t pl = size_t(b) * a.N;
+  const float* const vbar = a.vbar + size_t(b) * a.N * a.T;
   float lsum = 0.f;
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < N;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    const float ri = r[i], si = S[i];
-    double rsum = 0.0;
-    float fsum = 0.f;
-    // Frames in groups of kGroup with all loads of a group issued together
-    // (one memory latency per group); the sums keep frame order.
-    int t = 0;
-    for (; t + kGroup <= T; t += kGroup) {
-      float vb[kGroup], f[kGroup];
+  for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < n;
+       i += int64_t(gridDim.x) * kThreads) {
+    const Vec<V> ri = ldv<V>(a.r + b * a.r_b, i), si = ldv<V>(a.S, i);
+    Vec<V> yb = ldv<V>(a.ybar + pl, i), y1{};
+    if (a.y1bar_in) y1 = ldv<V>(a.y1bar_in + pl, i);
+    double rsum[V] = {};
+    float fsum[V] = {};
+    for (int t0 = 0; t0 < a.T; t0 += G) {
+      Vec<V> vb[G], f[G];
 #pragma unroll
-      for (int g = 0; g < kGroup; ++g) {
-        vb[g] = vbar[size_t(t + g) * N + i];
-        f[g] = phi[size_t(t + g) * N + i];
+      for (int g = 0; g < G; ++g) {
+        const int t = t0 + g < a.T ? t0 + g : a.T - 1;
+        vb[g] = ldv<V>(vbar + size_t(t) * a.N, i);
+        f[g] = ldv<V>(a.phi + size_t(t) * a.N, i);
       }
 #pragma unroll
-      for (int g = 0; g < kGroup; ++g) {
-        rsum = acc_prod(vb[g], f[g], rsum);
-        fsum += f[g];
+      for (int g = 0; g < G; ++g) {
+        if (t0 + g >= a.T) break;
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+          rsum[k] = acc_prod(vb[g].v[k], f[g].v[k], rsum[k]);
+          fsum[k] += f[g].v[k];
+        }
       }
     }
-    for (; t < T; ++t) {
-      const float vb = vbar[size_t(t) * N + i], f = phi[size_t(t) * N + i];
-      rsum = acc_prod(vb, f, rsum);
-      fsum += f;
+    Vec<V> y1o, ybb, sb;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      float rbar = float(rsum[k]);
+      lsum = fmaf(rbar, ri.v[k], lsum);  // dL/dlambda = sum_t vbar*r*Phi
+      rbar *= a.lam;
+      y1o.v[k] = y1.v[k] + rbar / si.v[k];
+      yb.v[k] += y1o.v[k];
+      ybb.v[k] = -rbar / si.v[k] - y1o.v[k];
+      // S = sum_t Phi_t, except where that sum is 0 and S is the constant 1.
+      sb.v[k] = fsum[k] != 0.f ? -rbar * ri.v[k] / si.v[k] : 0.f;
     }
-    float rbar = float(rsum);
-    lsum = fmaf(rbar, ri, lsum);  // dL/dlambda = sum_t vbar*r*Phi
-    rbar *= lam;
-    const float y1tot = (y1bar_ext ? y1bar_ext[i] : 0.f) + rbar / si;
-    y1bar_out[i] = y1tot;
-    ybar[i] += y1tot;
-    ybb_out[i] = -rbar / si - y1tot;
-    // S = sum_t Phi_t, except where that sum is 0 and S is the constant 1.
-    if (sbar_out) sbar_out[i] = fsum != 0.f ? -rbar * ri / si : 0.f;
+    stv<V>(a.y1bar_out + pl, i, y1o);
+    stv<V>(a.ybar + pl, i, yb);
+    stv<V>(a.ybb + pl, i, ybb);
+    if (a.sbar) stv<V>(a.sbar + pl, i, sb);
   }
-  block_atomic(lsum, lambar, 1.0);
+  block_atomic(lsum, a.lambar);
 }
 
-// Mask gradient of one projection: phibar_t += lambda r vbar_t + ybb x_t + Sbar.
-__global__ void __launch_bounds__(256) k_ub_phibar(
-    const float* __restrict__ vbar, const float* __restrict__ x, const float* __restrict__ r,
-    float lam, const float* __restrict__ ybb, const float* __restrict__ sbar,
-    float* __restrict__ phibar, int64_t N, int T) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < N;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    const float lr = lam * r[i], yb = ybb[i], sb = sbar[i];
-#pragma unroll kGroup
-    for (int t = 0; t < T; ++t) {
-      const size_t o = size_t(t) * N + i;
-      phibar[o] += fmaf(lr, vbar[o], fmaf(yb, x[o], sb));
+// Mask gradient of one projection: phibar_t += sum over the group's samples of
+// lambda r vbar_t + ybb x_t + Sbar.  One thread per pixel and frame
+// (blockIdx.y), one pass over phibar for the whole group.
+template <int V>
+__global__ void __launch_bounds__(kThreads) k_ub_phibar(
+    const float* __restrict__ vbar, const float* __restrict__ x, size_t x_b,
+    const float* __restrict__ r, size_t r_b, float lam, const float* __restrict__ ybb,
+    const float* __restrict__ sbar, float* __restrict__ phibar, int64_t N, int T, int nb) {
+  const int64_t n = N / V;
+  const size_t fr = size_t(blockIdx.y) * N;
+  for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < n;
+       i += int64_t(gridDim.x) * kThreads) {
+    Vec<V> acc = ldv<V>(phibar + fr, i);
+    for (int b = 0; b < nb; ++b) {
+      const size_t pl = size_t(b) * N;
+      const Vec<V> ri = ldv<V>(r + b * r_b, i), yb = ldv<V>(ybb + pl, i), sb = ldv<V>(sbar + pl, i);
+      const Vec<V> vb = ldv<V>(vbar + pl * T + fr, i), xv = ldv<V>(x + b * x_b + fr, i);
+#pragma unroll
+      for (int k = 0; k < V; ++k)
+        acc.v[k] += fmaf(lam * ri.v[k], vb.v[k], fmaf(yb.v[k], xv.v[k], sb.v[k]));
     }
+    stv<V>(phibar + fr, i, acc);
   }
 }
 
-// Reverse of x_0 = Phi*y: phibar += xbar_0 * y, ybar += sum_t xbar_0 * Phi,
-// with xbar_0 = vbar + ybb Phi formed here (ybb null: xbar_0 = vbar).
-__global__ void __launch_bounds__(256) k_ub_init(const float* __restrict__ vbar,
-                                                 const float* __restrict__ ybb,
-                                                 const float* __restrict__ phi,
-                                                 const float* __restrict__ y,
-                                                 float* __restrict__ ybar,
-                                                 float* __restrict__ phibar, int64_t N, int T) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < N;
-       i += int64_t(gridDim.x) * blockDim.x) {
+// End of the backward pass of a group.  Reverse of x_0 = Phi*y and, with
+// truth, of y = sum_t Phi_t truth_t: with xbar_0 = vbar + ybb Phi,
+//   ybar += sum_t xbar_0 Phi  (k_ub_end_y, blockIdx.y = sample),
+//   phibar += xbar_0 y (+ ybar truth)  (k_ub_end_phi, blockIdx.y = frame);
+// the last group writes the mask gradient itself (logits: times Phi (1 - Phi))
+// and the lambda and weight gradients from their slots.
+struct EndArgs {
+  const float* vbar;
+  const float* ybb;
+  const float* phi;
+  const float* y;
+  size_t y_b;
+  float* ybar;
+  float* phibar;
+  const float* truth;  // null: y was given
+  float* grad_mask;    // last group only, else null
+  int64_t N;
+  int T, nb, logits;
+  // last group only, else K = 0
+  const double* slots;
+  double* grad_lambda;
+  double* grad_weight;
+  int K;
+};
+
+__global__ void __launch_bounds__(kThreads) k_ub_end_y(EndArgs a) {
+  const int b = blockIdx.y;
+  const size_t pl = size_t(b) * a.N;
+  for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < a.N;
+       i += int64_t(gridDim.x) * kThreads) {
+    const float yb = a.ybb[pl + i];
     double acc = 0.0;
-    const float yv = y[i], yb = ybb ? ybb[i] : 0.f;
-#pragma unroll kGroup
-    for (int t = 0; t < T; ++t) {
-      const size_t o = size_t(t) * N + i;
-      const float f = phi[o];
-      const float xb = ybb ? fmaf(yb, f, vbar[o]) : vbar[o];
-      acc = acc_prod(xb, f, acc);
-      if (phibar) phibar[o] = fmaf(xb, yv, phibar[o]);
+#pragma unroll 8
+    for (int t = 0; t < a.T; ++t) {
+      const float f = a.phi[size_t(t) * a.N + i];
+      acc = acc_prod(fmaf(yb, f, a.vbar[pl * a.T + size_t(t) * a.N + i]), f, acc);
     }
-    ybar[i] += float(acc);
+    a.ybar[pl + i] += float(acc);
+  }
+  if (b == 0)  // lambda and weight gradient of iteration k: the sums of their slots
+    for (int k = blockIdx.x * kThreads + threadIdx.x; k < a.K; k += gridDim.x * kThreads) {
+      double gl = 0.0, gw = 0.0;
+      for (int j = 0; j < kGradSlots; ++j) {
+        gl += a.slots[(size_t(k) * 2 * kGradSlots + j) * kGradSlotStride];
+        gw += a.slots[((size_t(k) * 2 + 1) * kGradSlots + j) * kGradSlotStride];
+      }
+      a.grad_lambda[k] = gl;
+      a.grad_weight[k] = gw;
+    }
+}
+
+__global__ void __launch_bounds__(kThreads) k_ub_end_phi(EndArgs a) {
+  const size_t fr = size_t(blockIdx.y) * a.N;
+  for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < a.N;
+       i += int64_t(gridDim.x) * kThreads) {
+    const float f = a.phi[fr + i];
+    float g = a.phibar[fr + i];
+    for (int b = 0; b < a.nb; ++b) {
+      const size_t pl = size_t(b) * a.N, vo = pl * a.T + fr + i;
+      g = fmaf(fmaf(a.ybb[pl + i], f, a.vbar[vo]), a.y[b * a.y_b + i], g);
+      if (a.truth) g = fmaf(a.ybar[pl + i], a.truth[vo], g);
+    }
+    if (a.grad_mask)
+      a.grad_mask[fr + i] = a.logits ? g * f * (1.f - f) : g;
+    else
+      a.phibar[fr + i] = g;
   }
 }
 
-__global__ void k_fill_f32(float* p, int64_t n, float v) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * blockDim.x)
-    p[i] = v;
-}
-
-// dst += src (elementwise).
-__global__ void k_add_f32(float* __restrict__ dst, const float* __restrict__ src, int64_t n) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * blockDim.x)
-    dst[i] += src[i];
+// Zeroes of a backward pass in one launch.
+__global__ void k_zero(float* p, int64_t n, float* q, int64_t m, double* slots, int64_t ns) {
+  const int64_t first = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  const int64_t step = int64_t(gridDim.x) * blockDim.x;
+  for (int64_t i = first; i < n; i += step) p[i] = 0.f;
+  for (int64_t i = first; i < m; i += step) q[i] = 0.f;
+  for (int64_t i = first; i < ns; i += step) slots[i] = 0.0;
 }
 
 unsigned grid1(int64_t n) {
@@ -168,107 +269,204 @@ unsigned grid1(int64_t n) {
   return unsigned(b < 1 ? 1 : (b > 4096 ? 4096 : b));
 }
 
-// phi = sigmoid(logits).
-__global__ void k_sigmoid(const float* __restrict__ z, float* __restrict__ phi, int64_t n) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * blockDim.x)
-    phi[i] = 1.f / (1.f + expf(-z[i]));
-}
-
-// dL/dlogits = dL/dphi * phi * (1 - phi).
-__global__ void k_sigmoid_bwd(const float* __restrict__ phibar, const float* __restrict__ phi,
-                              float* __restrict__ zbar, int64_t n) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    const float f = phi[i];
-    zbar[i] = phibar[i] * f * (1.f - f);
+// phi = sigmoid(logits) when asked, and S = sum_t phi_t in frame order (a sum
+// of 0 becomes 1), as scigap_phi_sum forms it.
+__global__ void __launch_bounds__(kThreads) k_mask(const float* __restrict__ mask,
+                                                   float* __restrict__ phi,
+                                                   float* __restrict__ S, int64_t N, int T) {
+  for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < N;
+       i += int64_t(gridDim.x) * kThreads) {
+    float acc = 0.f;
+#pragma unroll 4
+    for (int t = 0; t < T; ++t) {
+      const size_t o = size_t(t) * N + i;
+      float f = mask[o];
+      if (phi) {
+        f = 1.f / (1.f + expf(-f));
+        phi[o] = f;
+      }
+      acc += f;
+    }
+    S[i] = acc == 0.f ? 1.f : acc;
   }
 }
 
-// Reverse of y = sum_t phi_t * truth_t: phibar_t += ybar * truth_t.
-__global__ void k_measure_bwd(const float* __restrict__ ybar, const float* __restrict__ truth,
-                              float* __restrict__ phibar, int64_t N, int T) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < N;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    const float yb = ybar[i];
-    for (int t = 0; t < T; ++t) phibar[size_t(t) * N + i] = fmaf(yb, truth[size_t(t) * N + i],
-                                                                 phibar[size_t(t) * N + i]);
+// Start of the forward pass, blockIdx.y = sample: y = sum_t Phi_t truth_t (or
+// the given measurement), x_0 = Phi y, yb = A x_0, y1 = y - yb,
+// r_0 = (y1 - yb)/S (the arithmetic of scigap_forward, scigap_adjoint and
+// k_init).
+struct StartArgs {
+  const float* meas;
+  int measure;
+  const float* phi;
+  const float* S;
+  float* y;
+  size_t y_b;
+  float* x0;
+  size_t x_b;
+  float* r;
+  size_t r_b;
+  float* y1;
+  size_t y1_b;
+  int64_t N;
+  int T;
+};
+
+__global__ void __launch_bounds__(kThreads) k_unrolled_start(StartArgs a) {
+  const int b = blockIdx.y;
+  const float* const meas = a.meas + size_t(b) * a.N * (a.measure ? a.T : 1);
+  for (int64_t i = blockIdx.x * int64_t(kThreads) + threadIdx.x; i < a.N;
+       i += int64_t(gridDim.x) * kThreads) {
+    float y;
+    if (a.measure) {
+      double acc = 0.0;
+#pragma unroll 4
+      for (int t = 0; t < a.T; ++t)
+        acc = acc_prod(meas[size_t(t) * a.N + i], a.phi[size_t(t) * a.N + i], acc);
+      y = float(acc);
+    } else {
+      y = meas[i];
+    }
+    a.y[b * a.y_b + i] = y;
+    double acc = 0.0;
+#pragma unroll 4
+    for (int t = 0; t < a.T; ++t) {
+      const float f = a.phi[size_t(t) * a.N + i];
+      const float x = y * f;
+      a.x0[b * a.x_b + size_t(t) * a.N + i] = x;
+      acc = acc_prod(x, f, acc);
+    }
+    const float yb = float(acc), y1 = y - yb;
+    a.y1[b * a.y1_b + i] = y1;
+    a.r[b * a.r_b + i] = (y1 - yb) / a.S[i];
   }
+}
+
+// Whether the per-pixel kernels take 4 pixels a lane: planes whose start and
+// distances keep 16-byte alignment, and enough of them (at 1024x1024x20 the
+// projection reverse takes 60-80 us with one pixel a lane; 4 pixels of a
+// 256x256 plane would leave 3 of 4 SIMDs without a wave).
+bool proj_vector(int64_t N, std::initializer_list<const void*> ptrs,
+                 std::initializer_list<size_t> dists) {
+  if (N % 4 != 0 || N < (int64_t(1) << 19)) return false;
+  for (const void* p : ptrs)
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+  for (size_t d : dists)
+    if (d % 4 != 0) return false;
+  return true;
 }
 
 }  // namespace
 
-int tv_backward_tiles(int D, const float* x, const float* phi, const float* r, float lam,
-                      const float* xbar, const float* ybb, float* vbar, int64_t H, int64_t W,
-                      int64_t T, float w, double* wbar, hipStream_t s);
+int tv_backward_tiles(int D, int nb, const float* x, size_t x_b, const float* phi, const float* r,
+                      size_t r_b, float lam, const float* xbar, size_t xbar_b, const float* ybb,
+                      size_t ybb_b, float* vbar, size_t vbar_b, int64_t H, int64_t W, int64_t T,
+                      float w, double* wbar, hipStream_t s);
 
-size_t unrolled_backward_workspace(int64_t H, int64_t W, int64_t T, int D) {
-  (void)D;
-  const size_t N = size_t(H) * W, V = N * size_t(T);
-  // vbar x2, y1bar x2, ybb x2, Sbar
-  return 2 * align256(V * 4) + 5 * align256(N * 4);
+namespace {
+
+// Scratch of the backward pass of a group of nb samples.
+struct BwdScratch {
+  float* vbar[2];
+  float* y1bar[2];
+  float* ybb[2];
+  float* sbar;
+  float* ybar;
+};
+
+size_t bwd_scratch(int64_t H, int64_t W, int64_t T, int nb, char* base, BwdScratch* out) {
+  const size_t N = size_t(H) * W * nb, V = N * size_t(T);
+  size_t off = 0;
+  auto take = [&](size_t n) {
+    float* q = base ? reinterpret_cast<float*>(base + off) : nullptr;
+    off += align256(n * 4);
+    return q;
+  };
+  BwdScratch b;
+  for (auto& p : b.vbar) p = take(V);
+  for (auto& p : b.y1bar) p = take(N);
+  for (auto& p : b.ybb) p = take(N);
+  b.sbar = take(N);
+  b.ybar = take(N);
+  if (out) *out = b;
+  return off;
 }
 
-// Backward through K unrolled iterations of one sample.
-int unrolled_backward(int64_t H, int64_t W, int64_t T, int K, int D, const float* lambdas,
-                      const float* weights, const float* y, const float* phi, const float* S,
-                      const float* ckpt_x, size_t xstride, const float* ckpt_r, size_t rstride,
-                      const float* grad_x,
-                      float* grad_phi, float* grad_y, double* grad_lambda, double* grad_weight,
-                      void* ws, hipStream_t s) {
-  const int64_t N = H * W, V = N * T;
-  char* base = static_cast<char*>(ws);
-  size_t off = 0;
-  auto take = [&](size_t bytes) {
-    char* q = base + off;
-    off += align256(bytes);
-    return reinterpret_cast<float*>(q);
-  };
-  float* vbar[2] = {take(V * 4), take(V * 4)};
-  float* y1bar[2] = {take(N * 4), take(N * 4)};
-  float* ybb[2] = {take(N * 4), take(N * 4)};
-  float* sbar = take(N * 4);
+// Where the forward pass left a group's samples (the first one's planes and
+// the distances to the next, in floats).
+struct GroupCkpt {
+  const float* x;
+  size_t xstride, x_b;
+  const float* r;
+  size_t rstride, r_b;
+  const float* y;
+  size_t y_b;
+};
 
-  k_fill_f32<<<grid1(N), 256, 0, s>>>(grad_y, N, 0.f);
-  SCIGAP_LAUNCH_CHECK("grad fill");
+// Backward through K unrolled iterations of nb samples.  phibar (null: no mask
+// gradient) accumulates; grad_mask, grad_lambda and grad_weight are written by
+// the last group.
+int unrolled_backward(int64_t H, int64_t W, int64_t T, int K, int D, int nb, const float* lambdas,
+                      const float* weights, const GroupCkpt& c, const float* phi, const float* S,
+                      const float* grad_x, const float* truth, float* phibar, float* grad_mask,
+                      int logits, bool last, double* slots, double* grad_lambda,
+                      double* grad_weight, const BwdScratch& w, hipStream_t s) {
+  const int64_t N = H * W;
+  const size_t V = size_t(N) * T;
   // Adjoint of x_{k+1}: grad_x for k = K-1, else vbar_{k+1} + ybb_{k+1} Phi
-  // (formed on load by the reverse TV step and by k_ub_init).
+  // (formed on load by the reverse TV step and by k_ub_end).
   const float* vb_in = grad_x;
   const float* ybb_in = nullptr;
   const float* y1b_in = nullptr;
   int sel = 0;
   for (int k = K - 1; k >= 0; --k) {
-    const float lam = lambdas[k], w = weights[k];
-    const float* xk = ckpt_x + size_t(k) * xstride;
-    const float* r = ckpt_r + size_t(k) * rstride;  // residual the forward used
+    const float lam = lambdas[k];
+    const float* xk = c.x + size_t(k) * c.xstride;
+    const float* r = c.r + size_t(k) * c.rstride;  // residual the forward used
     {
       ProfScope ps("unrolled_bwd_tv", s);
-      if (int rc = tv_backward_tiles(D, xk, phi, r, lam, vb_in, ybb_in, vbar[sel], H, W, T, w,
-                                     grad_weight + k, s))
+      if (int rc = tv_backward_tiles(D, nb, xk, c.x_b, phi, r, c.r_b, lam, vb_in, V, ybb_in,
+                                     size_t(N), w.vbar[sel], V, H, W, T, weights[k],
+                                     slots + size_t(2 * k + 1) * kGradSlots * kGradSlotStride, s))
         return rc;
     }
     {
       ProfScope ps("unrolled_bwd_proj", s);
-      k_ub_proj<<<grid1(N), 256, 0, s>>>(vbar[sel], phi, S, r, lam, y1b_in, y1bar[sel], grad_y,
-                                         ybb[sel], grad_phi ? sbar : nullptr, grad_lambda + k,
-                                         N, int(T));
+      ProjArgs a{w.vbar[sel], phi,         S,          r,     c.r_b, lam, y1b_in,
+                 w.y1bar[sel], w.ybar,     w.ybb[sel], phibar ? w.sbar : nullptr,
+                 slots + size_t(2 * k) * kGradSlots * kGradSlotStride, N, int(T)};
+      const bool vec = proj_vector(N, {a.vbar, phi, S, r, a.y1bar_in, a.y1bar_out, a.ybar, a.ybb,
+                                       a.sbar}, {c.r_b});
+      if (vec)
+        k_ub_proj<4, 4><<<dim3(grid1(N / 4), unsigned(nb)), kThreads, 0, s>>>(a);
+      else
+        k_ub_proj<1, 8><<<dim3(grid1(N), unsigned(nb)), kThreads, 0, s>>>(a);
       SCIGAP_LAUNCH_CHECK("unrolled projection backward");
-      if (grad_phi) {
-        k_ub_phibar<<<grid1(N), 256, 0, s>>>(vbar[sel], xk, r, lam, ybb[sel], sbar, grad_phi,
-                                             N, int(T));
+      if (phibar) {
+        const bool pv = vec && proj_vector(N, {xk, phibar}, {c.x_b});
+        if (pv)
+          k_ub_phibar<4><<<dim3(grid1(N / 4), unsigned(T)), kThreads, 0, s>>>(
+              w.vbar[sel], xk, c.x_b, r, c.r_b, lam, w.ybb[sel], w.sbar, phibar, N, int(T), nb);
+        else
+          k_ub_phibar<1><<<dim3(grid1(N), unsigned(T)), kThreads, 0, s>>>(
+              w.vbar[sel], xk, c.x_b, r, c.r_b, lam, w.ybb[sel], w.sbar, phibar, N, int(T), nb);
         SCIGAP_LAUNCH_CHECK("unrolled mask gradient");
       }
     }
-    vb_in = vbar[sel];
-    ybb_in = ybb[sel];
-    y1b_in = y1bar[sel];
+    vb_in = w.vbar[sel];
+    ybb_in = w.ybb[sel];
+    y1b_in = w.y1bar[sel];
     sel ^= 1;
   }
-  // x_0 = Phi * y
-  k_ub_init<<<grid1(N), 256, 0, s>>>(vb_in, ybb_in, phi, y, grad_y, grad_phi, N, int(T));
-  SCIGAP_LAUNCH_CHECK("unrolled init backward");
+  EndArgs e{vb_in, ybb_in, phi, c.y, c.y_b, w.ybar, phibar, truth, grad_mask, N, int(T), nb, logits,
+            slots, grad_lambda, grad_weight, last ? K : 0};
+  k_ub_end_y<<<dim3(grid1(N), unsigned(nb)), kThreads, 0, s>>>(e);
+  if (phibar) k_ub_end_phi<<<dim3(grid1(N), unsigned(T)), kThreads, 0, s>>>(e);
+  SCIGAP_LAUNCH_CHECK("unrolled backward end");
   return SCIGAP_OK;
 }
+
+}  // namespace
 
 }  // namespace scigap
 
@@ -278,12 +476,12 @@ int unrolled_backward(int64_t H, int64_t W, int64_t T, int K, int D, const float
 
 namespace scigap {
 
-int fill_f64(double* p, int n, double v, hipStream_t s);
-int unrolled_forward_iterations(int64_t H, int64_t W, int64_t T, int K, int D,
+int unrolled_forward_iterations(int64_t H, int64_t W, int64_t T, int K, int D, int nb,
                                 const float* lambdas, const float* weights, const float* y,
-                                const float* phi, const float* S, float* xs, size_t xstride,
-                                float* y1b, float* x_out, float* rs, size_t rstride,
-                                int* nexit, float* yb_part, hipStream_t s);
+                                size_t y_b, const float* phi, const float* S, float* xs,
+                                size_t xstride, size_t x_b, float* y1b, size_t y1_b,
+                                float* x_out, float* rs, size_t rstride, size_t r_b,
+                                float* yb_part, size_t part_b, hipStream_t s);
 
 namespace {
 
@@ -306,35 +504,27 @@ CkptLayout ckpt_layout(const scigap_unrolled& u) {
   return c;
 }
 
-// Samples of a batch run concurrently on up to kLanes streams ("lanes");
-// every lane has its own scratch, and lanes 1.. their own dL/dphi partial.
-constexpr int kLanes = 4;
-
-struct ULane {
-  float* y1b = nullptr;     // two y1 planes (forward)
-  int* nexit = nullptr;     // K
-  float* yb_part = nullptr; // [min(T,8)][H*W] partial yb of frame-split launches
-  float* ybar = nullptr;    // (H,W) dL/dy of one sample
-  float* phibar = nullptr;  // (T,H,W) dL/dphi partial (lanes >= 1)
-  void* bwd = nullptr;
-};
-
+// Workspace: the samples of a batch run in groups of up to kSamples, one
+// launch per step for the whole group.
 struct UWorkspace {
-  float* phi = nullptr;     // sigmoid(logits), when logits
-  float* S = nullptr;       // phi_sum
-  float* phibar = nullptr;  // (T,H,W) dL/dphi, when logits
-  double* gl = nullptr;     // K, when the caller passes no grad_lambda
-  double* gw = nullptr;     // K, when the caller passes no grad_weight
-  int lanes = 1;
-  ULane lane[kLanes];
+  float* phi = nullptr;      // sigmoid(logits), when logits
+  float* S = nullptr;        // phi_sum
+  float* phibar = nullptr;   // (T,H,W) dL/dphi
+  double* gl = nullptr;      // K, when the caller passes no grad_lambda
+  double* gw = nullptr;      // K, when the caller passes no grad_weight
+  double* slots = nullptr;   // [K][lambda, weight][kGradSlots] gradient accumulators
+  float* y1b = nullptr;      // two y1 planes per sample (forward)
+  float* yb_part = nullptr;  // [min(T,8)][H*W] per sample: partial yb of frame-split launches
+  size_t part_b = 0;
+  BwdScratch bwd;
   size_t bytes = 0;
 };
 
-int lanes_of(const scigap_unrolled& u) { return u.batch < kLanes ? u.batch : kLanes; }
+int group_of(const scigap_unrolled& u) { return u.batch < kSamples ? u.batch : kSamples; }
 
 UWorkspace carve(const scigap_unrolled& u, char* base) {
   const size_t N = size_t(u.H) * u.W, V = N * size_t(u.T), K = size_t(u.iters);
-  const int D = u.tv_iter_max - 1;
+  const size_t nb = size_t(group_of(u));
   UWorkspace w;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -344,92 +534,17 @@ UWorkspace carve(const scigap_unrolled& u, char* base) {
   };
   if (u.logits) w.phi = reinterpret_cast<float*>(take(V * 4));
   w.S = reinterpret_cast<float*>(take(N * 4));
-  if (u.logits) w.phibar = reinterpret_cast<float*>(take(V * 4));
+  w.phibar = reinterpret_cast<float*>(take(V * 4));
   w.gl = reinterpret_cast<double*>(take(K * 8));
   w.gw = reinterpret_cast<double*>(take(K * 8));
-  w.lanes = lanes_of(u);
-  for (int l = 0; l < w.lanes; ++l) {
-    ULane& L = w.lane[l];
-    L.y1b = reinterpret_cast<float*>(take(2 * N * 4));
-    L.nexit = reinterpret_cast<int*>(take(K * 4));
-    L.yb_part = reinterpret_cast<float*>(take(size_t(u.T < 8 ? u.T : 8) * N * 4));
-    L.ybar = reinterpret_cast<float*>(take(N * 4));
-    if (l > 0) L.phibar = reinterpret_cast<float*>(take(V * 4));
-    L.bwd = take(unrolled_backward_workspace(u.H, u.W, u.T, D));
-  }
-  w.bytes = off;
+  w.slots = reinterpret_cast<double*>(take(K * 2 * kGradSlots * kGradSlotStride * 8));
+  w.y1b = reinterpret_cast<float*>(take(2 * N * nb * 4));
+  w.part_b = size_t(u.T < 8 ? u.T : 8) * N;
+  w.yb_part = reinterpret_cast<float*>(take(w.part_b * nb * 4));
+  const size_t bw = bwd_scratch(u.H, u.W, u.T, int(nb), base ? base + off : nullptr, &w.bwd);
+  w.bytes = off + bw;
   return w;
 }
-
-// Non-blocking, default-priority streams for the lanes, created once per
-// device and kept for the life of the process.
-struct LanePool {
-  std::mutex mu;
-  std::map<int, std::vector<hipStream_t>> streams;
-};
-LanePool& lane_pool() {
-  static LanePool p;
-  return p;
-}
-
-// Fork: lanes 1.. of a call wait for everything enqueued on `s` so far.
-// Join: `s` waits for every lane.  With one lane, or while `s` is being
-// captured into a graph, all samples stay on `s` (no fork).
-class Lanes {
- public:
-  Lanes(int want, hipStream_t s) : s_(s) {
-    st_[0] = s;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (want <= 1 || hipStreamIsCapturing(s, &cs) != hipSuccess ||
-        cs != hipStreamCaptureStatusNone)
-      return;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return;
-    LanePool& p = lane_pool();
-    std::lock_guard<std::mutex> lock(p.mu);
-    std::vector<hipStream_t>& v = p.streams[dev];
-    while (int(v.size()) < kLanes - 1) {
-      hipStream_t t = nullptr;
-      if (hipStreamCreateWithFlags(&t, hipStreamNonBlocking) != hipSuccess) break;
-      v.push_back(t);
-    }
-    const int n = std::min<int>(want, 1 + int(v.size()));
-    if (n <= 1 || hipEventCreateWithFlags(&fork_, hipEventDisableTiming) != hipSuccess) return;
-    if (hipEventRecord(fork_, s) != hipSuccess) return;
-    for (int l = 1; l < n; ++l) {
-      if (hipStreamWaitEvent(v[l - 1], fork_, 0) != hipSuccess) return;
-      st_[l] = v[l - 1];
-      n_ = l + 1;
-    }
-  }
-  int count() const { return n_; }
-  hipStream_t stream(int l) const { return st_[l % n_]; }
-  int lane(int b) const { return b % n_; }
-  // Makes `s` wait for every lane; returns a status.
-  int join() {
-    for (int l = 1; l < n_; ++l) {
-      hipEvent_t e = nullptr;
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-        return fail(SCIGAP_EHIP, "hipEventCreate failed");
-      const bool ok = hipEventRecord(e, st_[l]) == hipSuccess &&
-                      hipStreamWaitEvent(s_, e, 0) == hipSuccess;
-      (void)hipEventDestroy(e);
-      if (!ok) return fail(SCIGAP_EHIP, "lane join failed");
-    }
-    n_ = 1;
-    return SCIGAP_OK;
-  }
-  ~Lanes() {
-    join();
-    if (fork_) (void)hipEventDestroy(fork_);
-  }
-
- private:
-  hipStream_t s_;
-  hipStream_t st_[kLanes] = {};
-  hipEvent_t fork_ = nullptr;
-  int n_ = 1;
-};
 
 int check_unrolled(const scigap_unrolled* u) {
   if (!u) return fail(SCIGAP_ENULL, "unrolled descriptor is NULL");
@@ -470,14 +585,11 @@ int check_common(const scigap_unrolled* u, const float* lambdas, const float* we
 // phi (from logits when asked) and its frame sum.
 int prepare_mask(const scigap_unrolled& u, const float* mask, const UWorkspace& w,
                  const float** phi, hipStream_t s) {
-  const int64_t N = u.H * u.W, V = N * u.T;
-  *phi = mask;
-  if (u.logits) {
-    k_sigmoid<<<grid1(V), 256, 0, s>>>(mask, w.phi, V);
-    SCIGAP_LAUNCH_CHECK("sigmoid launch");
-    *phi = w.phi;
-  }
-  return scigap_phi_sum(*phi, w.S, u.H, u.W, u.T, s);
+  const int64_t N = u.H * u.W;
+  *phi = u.logits ? w.phi : mask;
+  k_mask<<<grid1(N), kThreads, 0, s>>>(mask, u.logits ? w.phi : nullptr, w.S, N, int(u.T));
+  SCIGAP_LAUNCH_CHECK("mask launch");
+  return SCIGAP_OK;
 }
 
 }  // namespace
@@ -517,29 +629,24 @@ int scigap_unrolled_forward(const scigap_unrolled* u, const float* lambdas, cons
   const UWorkspace w = carve(*u, static_cast<char*>(workspace));
   const float* phi = nullptr;
   if (int rc = prepare_mask(*u, mask, w, &phi, s)) return rc;
-  Lanes lanes(w.lanes, s);  // sample b runs on lane b % lanes
-  for (int b = 0; b < u->batch; ++b) {
-    const ULane& L = w.lane[lanes.lane(b)];
-    hipStream_t ls = lanes.stream(b);
+  const size_t dist = cl.per_sample / 4;  // distance between samples in floats
+  for (int b = 0; b < u->batch; b += kSamples) {
+    const int nb = u->batch - b < kSamples ? u->batch - b : kSamples;
     char* cb = static_cast<char*>(ckpt) + cl.per_sample * b;
     float* xs = reinterpret_cast<float*>(cb + cl.x);
     float* rs = reinterpret_cast<float*>(cb + cl.r);
     float* yb = reinterpret_cast<float*>(cb + cl.y);
-    if (u->measure) {
-      if (int rc = scigap_forward(meas + size_t(b) * V, phi, yb, u->H, u->W, u->T, ls)) return rc;
-    } else {
-      hipError_t e = hipMemcpyAsync(yb, meas + size_t(b) * N, size_t(N) * 4,
-                                    hipMemcpyDeviceToDevice, ls);
-      if (e != hipSuccess) return hip_fail(e, "copy y");
-    }
-    if (int rc = scigap_adjoint(yb, phi, xs, u->H, u->W, u->T, ls)) return rc;  // x_0 = At(y)
-    if (int rc = unrolled_forward_iterations(u->H, u->W, u->T, u->iters, u->tv_iter_max - 1,
-                                             lambdas, weights, yb, phi, w.S, xs, cl.xstride,
-                                             L.y1b, x_out + size_t(b) * V, rs, cl.rstride,
-                                             L.nexit, L.yb_part, ls))
+    StartArgs a{meas + size_t(b) * (u->measure ? V : N), u->measure ? 1 : 0, phi, w.S, yb, dist, xs,
+                dist, rs, dist, w.y1b, size_t(2 * N), N, int(u->T)};
+    k_unrolled_start<<<dim3(grid1(N), unsigned(nb)), kThreads, 0, s>>>(a);
+    SCIGAP_LAUNCH_CHECK("unrolled start launch");
+    if (int rc = unrolled_forward_iterations(
+            u->H, u->W, u->T, u->iters, u->tv_iter_max - 1, nb, lambdas, weights, yb, dist, phi,
+            w.S, xs, cl.xstride, dist, w.y1b, size_t(2 * N), x_out + size_t(b) * V, rs, cl.rstride,
+            dist, w.yb_part, w.part_b, s))
       return rc;
   }
-  return lanes.join();
+  return SCIGAP_OK;
 }
 
 int scigap_unrolled_backward(const scigap_unrolled* u, const float* lambdas, const float* weights,
@@ -567,52 +674,31 @@ int scigap_unrolled_backward(const scigap_unrolled* u, const float* lambdas, con
   if (int rc = prepare_mask(*u, mask, w, &phi, s)) return rc;
   double* gl = grad_lambda ? grad_lambda : w.gl;
   double* gw = grad_weight ? grad_weight : w.gw;
-  if (int rc = fill_f64(gl, K, 0.0, s)) return rc;
-  if (int rc = fill_f64(gw, K, 0.0, s)) return rc;
-  float* phibar = grad_mask ? (u->logits ? w.phibar : grad_mask) : nullptr;
-  Lanes lanes(w.lanes, s);
-  // dL/dphi: lane 0 accumulates into phibar, lanes 1.. into their own
-  // partials, summed into phibar after the join.
-  float* lane_phibar[kLanes] = {phibar};
-  for (int l = 1; l < lanes.count(); ++l) lane_phibar[l] = phibar ? w.lane[l].phibar : nullptr;
-  if (phibar) {
-    for (int l = 0; l < lanes.count(); ++l) {
-      k_fill_f32<<<grid1(V), 256, 0, lanes.stream(l)>>>(lane_phibar[l], V, 0.f);
-      SCIGAP_LAUNCH_CHECK("gradient fill");
-    }
-  }
-  for (int b = 0; b < u->batch; ++b) {
-    const int l = lanes.lane(b);
-    const ULane& L = w.lane[l];
-    hipStream_t ls = lanes.stream(b);
-    float* pb = lane_phibar[l];
+  const size_t dist = cl.per_sample / 4;
+  const int group = group_of(*u);
+  float* const phibar = grad_mask ? w.phibar : nullptr;
+  for (int b = 0; b < u->batch; b += kSamples) {
+    const int nb = u->batch - b < kSamples ? u->batch - b : kSamples;
     const char* cb = static_cast<const char*>(ckpt) + cl.per_sample * b;
-    const float* xs = reinterpret_cast<const float*>(cb + cl.x);
-    const float* rs = reinterpret_cast<const float*>(cb + cl.r);
-    const float* yb = reinterpret_cast<const float*>(cb + cl.y);
-    if (int rc = unrolled_backward(u->H, u->W, u->T, K, D, lambdas, weights, yb, phi, w.S, xs,
-                                   cl.xstride, rs, cl.rstride, grad_x + size_t(b) * V, pb,
-                                   L.ybar, gl, gw, L.bwd, ls))
+    const GroupCkpt c{reinterpret_cast<const float*>(cb + cl.x), cl.xstride, dist,
+                      reinterpret_cast<const float*>(cb + cl.r), cl.rstride, dist,
+                      reinterpret_cast<const float*>(cb + cl.y), dist};
+    const bool first = b == 0, last = b + nb >= u->batch;
+    k_zero<<<grid1(first && phibar ? V : N * group), 256, 0, s>>>(
+        w.bwd.ybar, N * group, phibar, first && phibar ? V : 0, w.slots,
+        first ? int64_t(K) * 2 * kGradSlots * kGradSlotStride : 0);
+    SCIGAP_LAUNCH_CHECK("gradient fill");
+    if (int rc = unrolled_backward(u->H, u->W, u->T, K, D, nb, lambdas, weights, c, phi, w.S,
+                                   grad_x + size_t(b) * V,
+                                   u->measure ? meas + size_t(b) * V : nullptr, phibar,
+                                   last ? grad_mask : nullptr, u->logits, last, w.slots, gl, gw,
+                                   w.bwd, s))
       return rc;
-    if (u->measure && pb) {
-      k_measure_bwd<<<grid1(N), 256, 0, ls>>>(L.ybar, meas + size_t(b) * V, pb, N, int(u->T));
-      SCIGAP_LAUNCH_CHECK("measurement backward launch");
-    }
     if (!u->measure && grad_meas) {
-      hipError_t e = hipMemcpyAsync(grad_meas + size_t(b) * N, L.ybar, size_t(N) * 4,
-                                    hipMemcpyDeviceToDevice, ls);
+      hipError_t e = hipMemcpyAsync(grad_meas + size_t(b) * N, w.bwd.ybar, size_t(N) * nb * 4,
+                                    hipMemcpyDeviceToDevice, s);
       if (e != hipSuccess) return hip_fail(e, "copy dL/dy");
     }
-  }
-  const int nl = lanes.count();
-  if (int rc = lanes.join()) return rc;
-  for (int l = 1; l < nl && phibar; ++l) {
-    k_add_f32<<<grid1(V), 256, 0, s>>>(phibar, lane_phibar[l], V);
-    SCIGAP_LAUNCH_CHECK("gradient lane sum");
-  }
-  if (grad_mask && u->logits) {
-    k_sigmoid_bwd<<<grid1(V), 256, 0, s>>>(w.phibar, phi, grad_mask, V);
-    SCIGAP_LAUNCH_CHECK("sigmoid backward launch");
   }
   return SCIGAP_OK;
 }

@@ -132,4 +132,15 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Accumulators of a scalar gradient: the workgroups' atomic additions go to
+// kGradSlots slots on lines of their own and are summed at the end.  On one
+// address they serialise: 1024 of them made the projection reverse of
+// 4 x 256x256x8 take 17.8 us.
+constexpr int kGradSlots = 32;
+constexpr int kGradSlotStride = 16;  // doubles (one 128-byte line)
+__device__ __forceinline__ double* grad_slot(double* base) {
+  const unsigned b = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  return base + (b % kGradSlots) * kGradSlotStride;
+}
+
 }  // namespace scigap

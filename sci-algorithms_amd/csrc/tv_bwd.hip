@@ -66,11 +66,22 @@ struct BwdArgs {
                       // outer iteration, xbar = xbar + ybb * Phi formed on load
   const float* ybb;   // (H,W) or null (see xbar)
   float* vbar;        // (T,H,W) adjoint of the TV input
-  double* wbar;       // adjoint of the TV weight (accumulated)
+  double* wbar;       // adjoint of the TV weight (accumulated in its slots)
   int H, W, tiles_x, tiles_y;
   float tw;           // tau / w
   double wscale;      // dc/dw = -tau / w^2
+  // Samples of one launch and the distances between theirs (floats).
+  int nb;
+  size_t x_b, r_b, xbar_b, ybb_b, vbar_b;
 };
+
+__device__ __forceinline__ void select_sample(BwdArgs& a, int b) {
+  a.x += b * a.x_b;
+  a.r += b * a.r_b;
+  a.xbar += b * a.xbar_b;
+  if (a.ybb) a.ybb += b * a.ybb_b;
+  a.vbar += b * a.vbar_b;
+}
 
 struct BwdLds {
   float2 vimg[kBwdBY * kBwdRY * 64];  // v, [tile row][lane]
@@ -363,7 +374,7 @@ __device__ __forceinline__ void bwd_tile(const BwdArgs& a, int tile, int t, BwdL
   if (threadIdx.x == 0) {
     double tot = 0.0;
     for (int w = 0; w < kBwdBY; ++w) tot += L.red[w];
-    atomicAdd(a.wbar, tot * a.wscale);
+    atomicAdd(grad_slot(a.wbar), tot * a.wscale);
   }
 }
 
@@ -371,6 +382,7 @@ template <int D>
 __global__ void __launch_bounds__(64 * kBwdBY) k_tv_bwd(BwdArgs a) {
   __shared__ BwdLds L;
   const int tile = blockIdx.x, t = blockIdx.y;
+  select_sample(a, blockIdx.z);
   zero_exchange_edges(L);
   bwd_tile<D, true>(a, tile, t, L);
   bwd_tile<D, false>(a, tile, t, L);
@@ -381,7 +393,8 @@ int launch_tv_bwd(BwdArgs a, int T, hipStream_t s) {
   using G = BwdGeom<D>;
   a.tiles_x = tiles_across(a.W, G::LW, G::HC, G::OX);
   a.tiles_y = tiles_across(a.H, G::LH, G::HR, G::OY);
-  k_tv_bwd<D><<<dim3(unsigned(a.tiles_x * a.tiles_y), unsigned(T)), 64 * kBwdBY, 0, s>>>(a);
+  k_tv_bwd<D><<<dim3(unsigned(a.tiles_x * a.tiles_y), unsigned(T), unsigned(a.nb)), 64 * kBwdBY, 0,
+                s>>>(a);
   SCIGAP_LAUNCH_CHECK("fused TV backward launch");
   return SCIGAP_OK;
 }
@@ -515,7 +528,7 @@ struct BwdRows {
           A1[u][j][k] = a1;
           G0[k] = fmaf(kk, a[k], a0);
           G1[k] = fmaf(kk, b[k], a1);
-          ct = (k == 0 ? sp.owner : sp.own1 && sp.owner) ? fmaf(-nn, w, ct) : ct;
+          ct = fmaf(-nn, w, ct);  // 0 outside the image: no gradient there
         });
         // Row I - D - r adds to the weight's adjoint when the strip owns it:
         // rows [kHalo, kHalo + R), with I - D - r the strip's row.
@@ -537,16 +550,15 @@ struct BwdRows {
         }
       }
     });
-    cb += double(c);
+    cb += double(sp.owner ? c : 0.f);
     asm volatile("" : "+v"(cb));
   }
 };
 
 template <int D, bool EDGE>
-__device__ __forceinline__ double bwd_strip(const BwdSweepArgs& s, const Strip& st, int t) {
+__device__ __forceinline__ double bwd_strip(const BwdArgs& a, int R, const Strip& st, int t) {
   using E = BwdRows<D, EDGE>;
   constexpr int P = kBwdAhead, FILL = E::kFill, HALO = E::kHalo;
-  const BwdArgs& a = s.b;
   const int H = a.H, W = a.W, N = H * W;
   const StripPos& sp = st.sp;
   const int vo = (sp.row0 * W + sp.col) * 4;
@@ -562,7 +574,7 @@ __device__ __forceinline__ double bwd_strip(const BwdSweepArgs& s, const Strip& 
   f2 nx[P], nf[P], nb[P];
   f2 nr, ny, ng;  // read before or by other frames as well (Phi of xbar's row): one row ahead
   const float tw = a.tw, lam = a.lam;
-  const int rows_all = s.R + 2 * HALO;
+  const int rows_all = R + 2 * HALO;
   // Requests of step i: v's row i and xbar's row i - D + 1.
   auto request = [&](auto pc, int i) __attribute__((always_inline)) {
     constexpr int p = decltype(pc)::value % P;
@@ -596,8 +608,8 @@ __device__ __forceinline__ double bwd_strip(const BwdSweepArgs& s, const Strip& 
     __builtin_amdgcn_sched_barrier(0);
   });
 #pragma unroll 1
-  for (int b = 0; b < s.R; b += kRing) {
-    const bool last = b + kRing >= s.R;
+  for (int b = 0; b < R; b += kRing) {
+    const bool last = b + kRing >= R;
     static_for<kRing>([&](auto mc) __attribute__((always_inline)) {
       constexpr int m = decltype(mc)::value, I = FILL + m;
       constexpr int j = (I + kRing * 8 - HALO) % kRing;  // slot of the finished row
@@ -619,10 +631,12 @@ k_tv_bwd_sweep(BwdSweepArgs s) {
   const int item = tile_of_block(blockIdx.x, s.per_xcd) * kBwdWaves + w;
   double cb = 0.0;
   if (item < s.items) {
-    const int t = item / s.strips, strip = item - t * s.strips;
+    const int frame = item / s.strips, strip = item - frame * s.strips;
+    const int b = frame / s.T, t = frame - b * s.T;
+    select_sample(s.b, b);
     constexpr int HALO = 2 * D - 1;
     const Strip st(strip, s.strips_x, s.b.H, s.b.W, s.R, 2 * D, HALO, HALO);
-    cb = st.edge ? bwd_strip<D, true>(s, st, t) : bwd_strip<D, false>(s, st, t);
+    cb = st.edge ? bwd_strip<D, true>(s.b, s.R, st, t) : bwd_strip<D, false>(s.b, s.R, st, t);
   }
   // Weight adjoint: one double atomic per workgroup.
   cb = wave_sum(cb);
@@ -631,12 +645,12 @@ k_tv_bwd_sweep(BwdSweepArgs s) {
   if (threadIdx.x == 0) {
     double tot = 0.0;
     for (int k = 0; k < kBwdWaves; ++k) tot += red[k];
-    if (tot != 0.0) atomicAdd(s.b.wbar, tot * s.b.wscale);
+    if (tot != 0.0) atomicAdd(grad_slot(s.b.wbar), tot * s.b.wscale);
   }
 }
 
-// Rows a strip owns (see tv_sweep.hip): a strip of R rows costs about
-// R + 10 full rows, and a SIMD is about 2/3 busy with a single wave.
+// Rows a strip owns: a strip of R rows costs about R + 10 full rows; two waves
+// share a SIMD (D = 4), and one alone takes about 3/4 of the time of two.
 template <int D>
 int launch_tv_bwd_sweep(const BwdArgs& a, int T, hipStream_t s) {
   BwdSweepArgs g{};
@@ -645,16 +659,17 @@ int launch_tv_bwd_sweep(const BwdArgs& a, int T, hipStream_t s) {
   g.strips_x = tiles_across(a.W, 128, 2 * D, 128 - 4 * D);
   const double simds = device_simds();
   double best = 1e300;
-  for (int R : {8, 16, 32, 64}) {
-    const double waves = double(g.strips_x) * ((a.H + R - 1) / R) * T;
-    const double cost = std::max(1.5, std::ceil(waves / simds)) * (R + 10);
+  for (int R = 8; R <= 128; R += 8) {
+    const double waves = double(g.strips_x) * ((a.H + R - 1) / R) * T * a.nb;
+    const double n = std::ceil(waves / simds);
+    const double cost = (n + 0.5 * std::fmod(n, 2.0)) * (R + 10);
     if (cost < best * 0.999) {
       best = cost;
       g.R = R;
     }
   }
   g.strips = g.strips_x * ((a.H + g.R - 1) / g.R);
-  g.items = g.strips * T;
+  g.items = g.strips * T * a.nb;
   g.per_xcd = ((g.items + kBwdWaves - 1) / kBwdWaves + 7) / 8;
   k_tv_bwd_sweep<D><<<unsigned(g.per_xcd * 8), 64 * kBwdWaves, 0, s>>>(g);
   SCIGAP_LAUNCH_CHECK("TV backward sweep launch");
@@ -666,9 +681,11 @@ int launch_tv_bwd_sweep(const BwdArgs& a, int T, hipStream_t s) {
 // vbar = (d out_D / d v)^T xbar for every frame, and wbar += xbar . d out_D / dw,
 // for D fixed Chambolle updates with weight w on v = x + (lam r) Phi (D in
 // [1, 6]; H*W < 2^30 - 8).  With ybb non-null the adjoint is xbar + ybb*Phi.
-int tv_backward_tiles(int D, const float* x, const float* phi, const float* r, float lam,
-                      const float* xbar, const float* ybb, float* vbar, int64_t H, int64_t W,
-                      int64_t T, float w, double* wbar, hipStream_t s) {
+// nb samples; the pointers are the first one's, *_b the distances (floats).
+int tv_backward_tiles(int D, int nb, const float* x, size_t x_b, const float* phi, const float* r,
+                      size_t r_b, float lam, const float* xbar, size_t xbar_b, const float* ybb,
+                      size_t ybb_b, float* vbar, size_t vbar_b, int64_t H, int64_t W, int64_t T,
+                      float w, double* wbar, hipStream_t s) {
   BwdArgs a{};
   a.x = x;
   a.phi = phi;
@@ -680,6 +697,12 @@ int tv_backward_tiles(int D, const float* x, const float* phi, const float* r, f
   a.wbar = wbar;
   a.H = int(H);
   a.W = int(W);
+  a.nb = nb;
+  a.x_b = x_b;
+  a.r_b = r_b;
+  a.xbar_b = xbar_b;
+  a.ybb_b = ybb_b;
+  a.vbar_b = vbar_b;
   a.tw = float(0.25 / double(w));
   a.wscale = -double(kTauB) / (double(w) * double(w));
   switch (D) {
