@@ -66,6 +66,14 @@ int scigap_forward(const float* x, const float* phi, float* y,
 int scigap_adjoint(const float* y, const float* phi, float* x,
                    int64_t H, int64_t W, int64_t T, void* stream);
 
+/* The two operators on arrays in the reference's own (H,W,T) layout, with the
+ * results of scigap_forward/scigap_adjoint and no layout conversion.
+ * Replace A_/At_, PnP_SCI/python/utils.py:10-26. */
+int scigap_forward_hwt(const float* x, const float* phi, float* y,
+                       int64_t H, int64_t W, int64_t T, void* stream);
+int scigap_adjoint_hwt(const float* y, const float* phi, float* x,
+                       int64_t H, int64_t W, int64_t T, void* stream);
+
 /* phi_sum[h,w] = sum_t phi[t,h,w], with exact zeros replaced by 1.
  * Replaces pnp_sci_algo.py:491-492 (and pnp_sci_demo_kobe.py:77-78). */
 int scigap_phi_sum(const float* phi, float* phi_sum,

@@ -124,6 +124,179 @@ __global__ void __launch_bounds__(TT * 8) k_transpose(const float* __restrict__ 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Kernels on the reference's (H,W,T) layout.  A block takes P = blockDim.x
+// consecutive pixels, that is P*T consecutive floats: it moves them with
+// 16-byte accesses in memory order and hands them to the pixels (or frames)
+// through LDS, padded by one element every 32 so that reading with a stride
+// of T meets the banks evenly.
+//
+// All are bound by memory, or by their launch.  A_ plus At_ of 256x256x8 on
+// device tensors take 24 us; converting both operands first (six launches
+// instead of two, three times the traffic) they took 55.  A conversion of
+// 1024x1024x8 takes 12.5 us (5.4 TB/s, the rate of a copy); in 32x32 tiles, of
+// which 8 frames fill a quarter, 32.7.
+// ---------------------------------------------------------------------------
+
+__host__ __device__ inline int pad32(int e) { return e + (e >> 5); }
+
+// Pixels of a block for `bytes` of LDS per frame of a pixel: the most that
+// leave room for several blocks on a CU; 0 when not even one wave's pixels fit
+// (more than 120 frames of products, 240 of pixels): then each thread reads its
+// own pixel, or the 32x32 tiles of k_transpose run, which such frame counts fill.
+inline int hwt_pixels(int64_t T, int bytes) {
+  for (int P : {256, 128, 64})
+    if (int64_t(P) * T * bytes <= (P == 64 ? 60 : 40) * 1024) return P;
+  return 0;
+}
+inline size_t hwt_lds(int P, int64_t T, int bytes) {
+  return size_t(pad32(int(P * T)) + 1) * size_t(bytes);
+}
+
+// y = sum_t x_t * phi_t on (H,W,T) arrays: exact products in fp64, summed in
+// frame order (as k_forward).
+template <bool VEC>
+__global__ void __launch_bounds__(256) k_forward_hwt(const float* __restrict__ x,
+                                                     const float* __restrict__ phi,
+                                                     float* __restrict__ y, int64_t N, int T) {
+  extern __shared__ double prod[];
+  const int P = blockDim.x, tid = threadIdx.x;
+  const int64_t p0 = int64_t(blockIdx.x) * P;
+  const int64_t base = p0 * T;
+  const int n = int(p0 + P <= N ? P : N - p0) * T;
+  int done = 0;
+  if constexpr (VEC) {
+    const float4* const xv = reinterpret_cast<const float4*>(x + base);
+    const float4* const fv = reinterpret_cast<const float4*>(phi + base);
+    for (int i = tid; i < n / 4; i += P) {
+      const float4 a = xv[i], b = fv[i];
+      prod[pad32(4 * i)] = double(a.x) * double(b.x);
+      prod[pad32(4 * i + 1)] = double(a.y) * double(b.y);
+      prod[pad32(4 * i + 2)] = double(a.z) * double(b.z);
+      prod[pad32(4 * i + 3)] = double(a.w) * double(b.w);
+    }
+    done = n & ~3;
+  }
+  for (int i = done + tid; i < n; i += P)
+    prod[pad32(i)] = double(x[base + i]) * double(phi[base + i]);
+  __syncthreads();
+  if (p0 + tid < N) {
+    double s = 0.0;
+    for (int t = 0; t < T; ++t) s += prod[pad32(tid * T + t)];
+    y[p0 + tid] = float(s);
+  }
+}
+
+// The same for frame counts whose products do not fit the LDS.
+__global__ void __launch_bounds__(kThreads) k_forward_hwt_many(const float* __restrict__ x,
+                                                               const float* __restrict__ phi,
+                                                               float* __restrict__ y, int64_t N,
+                                                               int T) {
+  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < N;
+       i += int64_t(gridDim.x) * blockDim.x) {
+    double s = 0.0;
+    for (int t = 0; t < T; ++t) s = acc_prod(x[i * T + t], phi[i * T + t], s);
+    y[i] = float(s);
+  }
+}
+
+// x_t = y * phi_t on (H,W,T) arrays; 256 pixels a block.
+template <bool VEC>
+__global__ void __launch_bounds__(kThreads) k_adjoint_hwt(const float* __restrict__ y,
+                                                          const float* __restrict__ phi,
+                                                          float* __restrict__ x, int64_t N,
+                                                          int T) {
+  __shared__ float ys[kThreads];
+  const int64_t p0 = int64_t(blockIdx.x) * kThreads;
+  const int tid = threadIdx.x;
+  const int64_t base = p0 * T;
+  const int64_t n = (p0 + kThreads <= N ? kThreads : N - p0) * int64_t(T);
+  if (p0 + tid < N) ys[tid] = y[p0 + tid];
+  __syncthreads();
+  int64_t done = 0;
+  if constexpr (VEC) {
+    const float4* const fv = reinterpret_cast<const float4*>(phi + base);
+    float4* const xv = reinterpret_cast<float4*>(x + base);
+    for (unsigned i = tid; i < unsigned(n / 4); i += kThreads) {
+      const float4 f = fv[i];
+      unsigned p = 4 * i / unsigned(T), r = 4 * i - p * unsigned(T);
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[k] = ys[p];
+        if (++r == unsigned(T)) {
+          r = 0;
+          p = p < kThreads - 1 ? p + 1 : p;
+        }
+      }
+      xv[i] = make_float4(v[0] * f.x, v[1] * f.y, v[2] * f.z, v[3] * f.w);
+    }
+    done = n & ~int64_t(3);
+  }
+  for (int64_t i = done + tid; i < n; i += kThreads) x[base + i] = ys[i / T] * phi[base + i];
+}
+
+// (H,W,T) <-> (T,H,W).  FROM_HWT: src is (H,W,T).  Vector accesses on both
+// sides (host: N % 4 == 0, 16-byte pointers), full blocks only; the last block
+// and other shapes go element by element.
+template <bool FROM_HWT, bool VEC>
+__global__ void __launch_bounds__(256) k_relayout(const float* __restrict__ src,
+                                                  float* __restrict__ dst, int64_t N, int T) {
+  extern __shared__ float buf[];
+  const int P = blockDim.x, tid = threadIdx.x;
+  const int64_t p0 = int64_t(blockIdx.x) * P, base = p0 * T;
+  const int np = int(p0 + P <= N ? P : N - p0), n = np * T;
+  const bool vec = VEC && np == P;
+  const int shift = __builtin_ctz(P) - 2;  // P/4 = 1 << shift
+  if constexpr (FROM_HWT) {
+    if (vec) {
+      const float4* const v = reinterpret_cast<const float4*>(src + base);
+      for (int i = tid; i < n / 4; i += P) {
+        const float4 a = v[i];
+        buf[pad32(4 * i)] = a.x;
+        buf[pad32(4 * i + 1)] = a.y;
+        buf[pad32(4 * i + 2)] = a.z;
+        buf[pad32(4 * i + 3)] = a.w;
+      }
+    } else {
+      for (int i = tid; i < n; i += P) buf[pad32(i)] = src[base + i];
+    }
+    __syncthreads();
+    if (vec) {
+      for (int i = tid; i < n / 4; i += P) {
+        const int t = i >> shift, q = 4 * (i & ((1 << shift) - 1));
+        reinterpret_cast<float4*>(dst + t * N + p0)[q >> 2] =
+            make_float4(buf[pad32(q * T + t)], buf[pad32((q + 1) * T + t)],
+                        buf[pad32((q + 2) * T + t)], buf[pad32((q + 3) * T + t)]);
+      }
+    } else if (tid < np) {
+      for (int t = 0; t < T; ++t) dst[t * N + p0 + tid] = buf[pad32(tid * T + t)];
+    }
+  } else {
+    if (vec) {
+      for (int i = tid; i < n / 4; i += P) {
+        const int t = i >> shift, q = 4 * (i & ((1 << shift) - 1));
+        const float4 a = reinterpret_cast<const float4*>(src + t * N + p0)[q >> 2];
+        buf[pad32(q * T + t)] = a.x;
+        buf[pad32((q + 1) * T + t)] = a.y;
+        buf[pad32((q + 2) * T + t)] = a.z;
+        buf[pad32((q + 3) * T + t)] = a.w;
+      }
+    } else if (tid < np) {
+      for (int t = 0; t < T; ++t) buf[pad32(tid * T + t)] = src[t * N + p0 + tid];
+    }
+    __syncthreads();
+    if (vec) {
+      float4* const v = reinterpret_cast<float4*>(dst + base);
+      for (int i = tid; i < n / 4; i += P)
+        v[i] = make_float4(buf[pad32(4 * i)], buf[pad32(4 * i + 1)], buf[pad32(4 * i + 2)],
+                           buf[pad32(4 * i + 3)]);
+    } else {
+      for (int i = tid; i < n; i += P) dst[base + i] = buf[pad32(i)];
+    }
+  }
+}
+
 __global__ void k_fill_f64(double* p, int n, double v) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -279,11 +452,85 @@ int scigap_phi_sum(const float* phi, float* phi_sum, int64_t H, int64_t W, int64
   return SCIGAP_OK;
 }
 
+int scigap_forward_hwt(const float* x, const float* phi, float* y, int64_t H, int64_t W, int64_t T,
+                       void* stream) {
+  clear_error();
+  if (int rc = check_shape(H, W, T)) return rc;
+  if (!x || !phi || !y) return fail(SCIGAP_ENULL, "scigap_forward_hwt: null pointer");
+  const int64_t N = H * W;
+  if (overlaps(y, N * 4, x, N * T * 4) || overlaps(y, N * 4, phi, N * T * 4))
+    return fail(SCIGAP_EALIAS, "scigap_forward_hwt: y overlaps an input");
+  hipStream_t s = as_stream(stream);
+  const int P = hwt_pixels(T, 8);
+  if (P == 0) {
+    k_forward_hwt_many<<<grid_for(N), kThreads, 0, s>>>(x, phi, y, N, int(T));
+  } else {
+    const unsigned blocks = unsigned((N + P - 1) / P);
+    const bool vec =
+        (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(phi)) % 16 == 0;
+    if (vec)
+      k_forward_hwt<true><<<blocks, P, hwt_lds(P, T, 8), s>>>(x, phi, y, N, int(T));
+    else
+      k_forward_hwt<false><<<blocks, P, hwt_lds(P, T, 8), s>>>(x, phi, y, N, int(T));
+  }
+  SCIGAP_LAUNCH_CHECK("scigap_forward_hwt launch");
+  return SCIGAP_OK;
+}
+
+int scigap_adjoint_hwt(const float* y, const float* phi, float* x, int64_t H, int64_t W, int64_t T,
+                       void* stream) {
+  clear_error();
+  if (int rc = check_shape(H, W, T)) return rc;
+  if (!x || !phi || !y) return fail(SCIGAP_ENULL, "scigap_adjoint_hwt: null pointer");
+  const int64_t N = H * W;
+  if (overlaps(x, N * T * 4, y, N * 4) || overlaps(x, N * T * 4, phi, N * T * 4))
+    return fail(SCIGAP_EALIAS, "scigap_adjoint_hwt: x overlaps an input");
+  hipStream_t s = as_stream(stream);
+  const unsigned blocks = unsigned((N + kThreads - 1) / kThreads);
+  const bool vec = (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(phi)) % 16 == 0;
+  if (vec)
+    k_adjoint_hwt<true><<<blocks, kThreads, 0, s>>>(y, phi, x, N, int(T));
+  else
+    k_adjoint_hwt<false><<<blocks, kThreads, 0, s>>>(y, phi, x, N, int(T));
+  SCIGAP_LAUNCH_CHECK("scigap_adjoint_hwt launch");
+  return SCIGAP_OK;
+}
+
+// (H,W,T) <-> (T,H,W) through k_relayout; false when T does not fit its LDS.
+static bool relayout(bool from_hwt, const float* src, float* dst, int64_t N, int64_t T,
+                     hipStream_t s) {
+  const int P = hwt_pixels(T, 4);
+  if (P == 0) return false;
+  const unsigned blocks = unsigned((N + P - 1) / P);
+  const size_t lds = hwt_lds(P, T, 4);
+  const bool vec = N % 4 == 0 &&
+                   (reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) % 16 == 0;
+  if (from_hwt) {
+    if (vec)
+      k_relayout<true, true><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+    else
+      k_relayout<true, false><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+  } else {
+    if (vec)
+      k_relayout<false, true><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+    else
+      k_relayout<false, false><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+  }
+  return true;
+}
+
 static int transpose(const float* src, float* dst, int64_t rows, int64_t cols, void* stream,
                      const char* name) {
   if (!src || !dst) return fail(SCIGAP_ENULL, "%s: null pointer", name);
   if (overlaps(src, rows * cols * 4, dst, rows * cols * 4))
     return fail(SCIGAP_EALIAS, "%s: src and dst overlap", name);
+  // One side of the matrix is the frame axis: rows = H*W for (H,W,T) -> (T,H,W).
+  const bool from_hwt = rows >= cols;
+  if (relayout(from_hwt, src, dst, from_hwt ? rows : cols, from_hwt ? cols : rows,
+               as_stream(stream))) {
+    SCIGAP_LAUNCH_CHECK(name);
+    return SCIGAP_OK;
+  }
   int64_t gx = (cols + TT - 1) / TT, gy = (rows + TT - 1) / TT;
   if (gx > (int64_t(1) << 31) - 1) return fail(SCIGAP_EINVAL, "%s: volume too large", name);
   if (gy > 65535) gy = 65535;

@@ -100,6 +100,8 @@ SYMBOLS = {
     "scigap_last_error": (ctypes.c_char_p, []),
     "scigap_forward": (_INT, [_P, _P, _P, _I64, _I64, _I64, _P]),
     "scigap_adjoint": (_INT, [_P, _P, _P, _I64, _I64, _I64, _P]),
+    "scigap_forward_hwt": (_INT, [_P, _P, _P, _I64, _I64, _I64, _P]),
+    "scigap_adjoint_hwt": (_INT, [_P, _P, _P, _I64, _I64, _I64, _P]),
     "scigap_phi_sum": (_INT, [_P, _P, _I64, _I64, _I64, _P]),
     "scigap_hwt_to_thw": (_INT, [_P, _P, _I64, _I64, _I64, _P]),
     "scigap_thw_to_hwt": (_INT, [_P, _P, _I64, _I64, _I64, _P]),

@@ -138,6 +138,17 @@ def to_host_like(t, like):
     return t.cpu().numpy().astype(dt, copy=False)
 
 
+def is_frame_major(a) -> bool:
+    """True for the NumPy (H,W,T) arrays that `to_device_thw` uploads as they
+    lie: C-ordered as (T,H,W) or, Fortran-ordered, as (T,W,H)."""
+    if is_torch(a):
+        return False
+    arr = np.asarray(a)
+    return (arr.ndim == 3 and arr.dtype.kind in "fiub"
+            and (arr.transpose(2, 0, 1).flags.c_contiguous
+                 or arr.transpose(2, 1, 0).flags.c_contiguous))
+
+
 def to_device_thw(a, name: str = "array"):
     """Frame-major (T,H,W) float32 device copy of an (H,W,T) array.
 

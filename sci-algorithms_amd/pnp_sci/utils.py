@@ -11,7 +11,7 @@ from __future__ import annotations
 import math
 
 from . import _lib
-from .device import thw_to_hwt, to_device, to_device_thw, to_host_like, sq_error
+from .device import is_frame_major, thw_to_hwt, to_device, to_device_thw, to_host_like, sq_error
 
 __all__ = ["A_", "At_", "psnr", "make_operators", "SCIOperator"]
 
@@ -22,8 +22,21 @@ def _torch():
 
 
 def A_(x, Phi):
-    """y[h,w] = sum_t x[h,w,t]*Phi[h,w,t]  (utils.py:10-15) via scigap_forward."""
+    """y[h,w] = sum_t x[h,w,t]*Phi[h,w,t]  (utils.py:10-15) via scigap_forward_hwt,
+    or scigap_forward where an operand is frame-major in memory already."""
     torch = _torch()
+    if not (is_frame_major(x) or is_frame_major(Phi)):
+        xd = to_device(x, "x")
+        pd = to_device(Phi, "Phi")
+        H, W, T = pd.shape
+        if tuple(xd.shape) != (H, W, T):
+            raise ValueError("x and Phi shapes differ: %s vs %s"
+                             % (tuple(x.shape), tuple(Phi.shape)))
+        y = torch.empty((H, W), dtype=torch.float32, device=xd.device)
+        L = _lib.lib()
+        _lib.check(L.scigap_forward_hwt(xd.data_ptr(), pd.data_ptr(), y.data_ptr(), H, W, T,
+                                        _lib.stream_ptr()))
+        return to_host_like(y, x)
     xd = to_device_thw(x, "x")
     pd = to_device_thw(Phi, "Phi")
     T, H, W = pd.shape
@@ -37,9 +50,21 @@ def A_(x, Phi):
 
 
 def At_(y, Phi):
-    """x[h,w,t] = y[h,w]*Phi[h,w,t]  (utils.py:17-26) via scigap_adjoint."""
+    """x[h,w,t] = y[h,w]*Phi[h,w,t]  (utils.py:17-26) via scigap_adjoint_hwt,
+    or scigap_adjoint where Phi is frame-major in memory already."""
     torch = _torch()
     yd = to_device(y, "y")
+    if not is_frame_major(Phi):
+        pd = to_device(Phi, "Phi")
+        H, W, T = pd.shape
+        if tuple(yd.shape) != (H, W):
+            raise ValueError("y shape %s does not match Phi %s"
+                             % (tuple(y.shape), tuple(Phi.shape)))
+        x = torch.empty((H, W, T), dtype=torch.float32, device=yd.device)
+        L = _lib.lib()
+        _lib.check(L.scigap_adjoint_hwt(yd.data_ptr(), pd.data_ptr(), x.data_ptr(), H, W, T,
+                                        _lib.stream_ptr()))
+        return to_host_like(x, y)
     pd = to_device_thw(Phi, "Phi")
     T, H, W = pd.shape
     if tuple(yd.shape) != (H, W):
