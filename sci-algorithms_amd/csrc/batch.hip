@@ -14,8 +14,9 @@
 //    the most frames come first (longest-processing-time order);
 //  * one workgroup per CU pulls items from its XCD's queue with an atomic
 //    counter and steals from the other queues when its own is drained;
-//  * interior and border tiles share the launch (the border body is chosen
-//    per item, encoded as a negative tile index);
+//  * interior and border tiles share the launch (the main pass chooses its
+//    body per strip; the repair's is chosen per item, a border tile having a
+//    negative index);
 //  * the early-exit decision and repair run per solve after every iteration;
 //  * with use_graph the whole run (counter resets, init, every iteration,
 //    ADMM's final projection) is captured once as a hipGraph and replayed.
@@ -58,10 +59,7 @@ k_fused_batch(const FusedArgs* __restrict__ descs, const int2* __restrict__ queu
       __syncthreads();
       if (q >= cnt) break;
       const int2 it = queue[beg + q];
-      if (it.y >= 0)
-        fused_tile<D, BY, MR, MODE, true, false>(descs[it.x], it.y, sh);
-      else
-        fused_tile<D, BY, MR, MODE, false, false>(descs[it.x], ~it.y, sh);
+      fused_tile<D, BY, MR, MODE, false>(descs[it.x], it.y >= 0 ? it.y : ~it.y, sh);
       __syncthreads();
     }
   }

@@ -83,50 +83,36 @@ __device__ __forceinline__ void st1(float* p, int N, unsigned o, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), plane_rsrc(p, N), o * 4u, 0, 0);
 }
 
-// Load an RY x 2 register block of one plane (zero outside the image).
-// `off` is the plane offset of register (0,0).  INSIDE tiles lie entirely in
-// the image (and W is even): one 8-byte buffer load per row (a wave reads 512
-// contiguous bytes per instruction), the row step in the scalar offset.
-// Border tiles send pixels outside the image to an offset past the end of
-// the buffer, which reads as 0.
-template <int RY, bool INSIDE>
-__device__ __forceinline__ void load_plane(const float* __restrict__ src, float (&v)[RY][2],
-                                           const LanePos& lp, int off, int H, int W) {
-  const __amdgpu_buffer_rsrc_t rs = plane_rsrc(src, H * W);
-  if constexpr (INSIDE) {
-    const int vo = off * 4;
-#pragma unroll
-    for (int j = 0; j < RY; ++j) {
-      const buffer_f2 f = raw_buffer_load_f2(rs, vo, j * W * 4, 0);
-      v[j][0] = f.x;
-      v[j][1] = f.y;
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < RY; ++j) {
-      const int r = lp.row0 + j;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int c = lp.col + k;
-        const bool in = r >= 0 && r < H && c >= 0 && c < W;
-        const unsigned o = in ? unsigned(off + j * W + k) * 4u : 0xFFFFFFF0u;
-        v[j][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0));
-      }
-    }
-  }
-}
+// How a strip's pixels lie in the image.
+enum Cover {
+  COVER_NONE = 0,  // rows and columns may lie outside
+  COVER_COLS = 1,  // every column inside, rows may lie outside
+  COVER_ALL = 2,   // every pixel inside
+};
 
-// Row j of load_plane alone.
-template <int RY, bool INSIDE>
+// Row j of an RY x 2 register block of one plane (zero outside the image).
+// `off` is the plane offset of register (0,0).  Strips whose columns all lie
+// in the image take one 8-byte buffer load per row (a wave reads 512 contiguous
+// bytes per instruction; buffer loads need 4-byte alignment only, so W may be
+// odd), the row step in the scalar offset where the rows do too.  Otherwise
+// pixels outside the image go to an offset past the end of the buffer, which
+// reads as 0, with one load per pixel where the columns need it.
+template <int RY, int COVER>
 __device__ __forceinline__ void load_row(const float* __restrict__ src, float (&v)[RY][2],
                                          const LanePos& lp, int off, int H, int W, int j) {
   const __amdgpu_buffer_rsrc_t rs = plane_rsrc(src, H * W);
-  if constexpr (INSIDE) {
+  const int r = lp.row0 + j;
+  if constexpr (COVER == COVER_ALL) {
     const buffer_f2 f = raw_buffer_load_f2(rs, off * 4, j * W * 4, 0);
     v[j][0] = f.x;
     v[j][1] = f.y;
+  } else if constexpr (COVER == COVER_COLS) {
+    const bool in = r >= 0 && r < H;
+    const buffer_f2 f =
+        raw_buffer_load_f2(rs, int(in ? unsigned(off + j * W) * 4u : 0xFFFFFFF0u), 0, 0);
+    v[j][0] = f.x;
+    v[j][1] = f.y;
   } else {
-    const int r = lp.row0 + j;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int c = lp.col + k;
@@ -135,6 +121,13 @@ __device__ __forceinline__ void load_row(const float* __restrict__ src, float (&
       v[j][k] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0));
     }
   }
+}
+
+template <int RY, int COVER>
+__device__ __forceinline__ void load_plane(const float* __restrict__ src, float (&v)[RY][2],
+                                           const LanePos& lp, int off, int H, int W) {
+#pragma unroll
+  for (int j = 0; j < RY; ++j) load_row<RY, COVER>(src, v, lp, off, H, W, j);
 }
 
 // Dual updates over which the requests for the next frame's Phi and x are
@@ -212,11 +205,13 @@ struct TilePlace {
   bool lane_owner; // lane's columns are interior columns of the tile
   bool own_c[2];   // interior column inside the image
   unsigned own_r;  // bit j: row0+j is an interior row inside the image
-  __device__ TilePlace(int tile, int tiles_x, int H, int W) {
+  __device__ TilePlace(int tile, int tiles_x, int H, int W)
+      : TilePlace(tile, tiles_x, H, W, int(threadIdx.x >> 6)) {}
+  __device__ TilePlace(int tile, int tiles_x, int H, int W, int strip) {
     const int ty = tile / tiles_x, tx = tile - ty * tiles_x;
     const ColPlace cp = col_place(tx, tiles_x, W, G::LW, G::HC, G::OX);
     const int c0 = cp.c0, r0 = ty * G::OY - D;
-    lp.w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lp.w = __builtin_amdgcn_readfirstlane(strip);
     lp.lane = threadIdx.x & 63;
     lp.row0 = r0 + lp.w * G::RY;
     lp.col = c0 + 2 * lp.lane;
@@ -263,8 +258,7 @@ __device__ __forceinline__ void commit_err(float err, double* dst, double* red64
   }
 }
 
-// Main pass.  INSIDE selects the interior tiles (no masks, no bounds checks)
-// or the border ring; IQA adds the squared error against the truth.
+// Main pass; IQA adds the squared error against the truth.
 // Registers hold the stencil state (out, p0, p1), lambda*r, the current Phi,
 // the yb accumulator and the prefetched next frame (x, Phi); the TV input
 // img lives in LDS as a [tile row][128] float plane (the engine reads it on
@@ -336,22 +330,22 @@ __device__ __forceinline__ void store_owned(float* __restrict__ p, int N, int W,
   }
 }
 
-// One tile of one fused outer iteration (the body of k_fused and of the
-// batched persistent kernel).  Returns without work when the tile's class
-// (interior/border) differs from INSIDE.  X1 selects the one-barrier TV
+// One strip (wave) of one tile of one fused outer iteration.  X1 selects the one-barrier TV
 // engine (tv_run_x1).  ENERGY false: no exit test follows and no energies are
 // formed.
-template <int D, int BY, int MR, int MODE, bool INSIDE, bool IQA, bool X1 = false,
-          bool DMA = false, bool ENERGY = true>
-__device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
-                                           FusedLds<D, BY, MR, X1, DMA>& sh, int part = 0) {
+template <int D, int BY, int MR, int MODE, Cover COVER, Edge EDGE, bool IQA, bool X1, bool DMA, bool ENERGY,
+          StripKind STRIP>
+__device__ __forceinline__ void fused_strip(const FusedArgs& a, int tile,
+                                            FusedLds<D, BY, MR, X1, DMA>& sh, int part,
+                                            int strip) {
+  constexpr bool INSIDE = COVER == COVER_ALL;
+  constexpr bool kOwn = STRIP == STRIP_OWN;  // else a halo strip: owns no row
   using G = TileGeom<D, BY, MR>;
   constexpr int RY = G::RY;
   constexpr int NH = MR;
   // Interior tiles may prefetch the next frame straight into LDS.
-  constexpr bool kDma = DMA && INSIDE && (RY % 2 == 0);
+  constexpr bool kDma = DMA && EDGE == EDGE_NONE && (RY % 2 == 0);
   auto& lds = sh.eng;
-  if constexpr (!X1) lds.zero_edges();
   float* const red = sh.red;
   double* const red64 = sh.red64;
   const int H = a.H, W = a.W;
@@ -360,15 +354,15 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
   const int nparts = a.fsplit > 1 ? a.fsplit : 1;
   const int t_lo = (a.T * part) / nparts;
   const int T = (a.T * (part + 1)) / nparts - t_lo;
-  const TilePlace<D, BY, MR> tp(tile, a.tiles_x, H, W);
-  if (tp.inside != INSIDE) return;
+  const TilePlace<D, BY, MR> tp(tile, a.tiles_x, H, W, strip);
   const LanePos& lp = tp.lp;
   const int off0 = tp.off0;
   // LDS slot of register row j of this lane: (w*RY + j)*64 + lane.
   const int sl0 = lp.w * RY * 64 + lp.lane;
 
   EdgeMasks em;
-  if constexpr (!INSIDE) em.init<RY>(lp, H, W);
+  if constexpr (EDGE == EDGE_ANY) em.init<RY>(lp, H, W);
+  if constexpr (EDGE == EDGE_RIGHT) em.init_right(lp, W);
 
   const bool from_y = a.from_y;
   // q = lambda*r (or y + lambda*r when X_0 = At(y)) over the load tile.
@@ -386,10 +380,10 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
   double* ybl = nullptr;
   if constexpr (kYbInLds) ybl = sh.ybs.v + size_t(sl0) * 2;  // row j at ybl[j * 128]
   if constexpr (MODE != TV_ONLY) {
-    load_plane<RY, INSIDE>(a.r_in, q, lp, off0, H, W);
+    load_plane<RY, COVER>(a.r_in, q, lp, off0, H, W);
     if (from_y) {
       float yv[RY][2];
-      load_plane<RY, INSIDE>(a.y, yv, lp, off0, H, W);
+      load_plane<RY, COVER>(a.y, yv, lp, off0, H, W);
 #pragma unroll
       for (int j = 0; j < RY; ++j)
 #pragma unroll
@@ -401,7 +395,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
         for (int k = 0; k < 2; ++k) q[j][k] *= a.lam;
     }
   }
-  if constexpr (MODE != TV_ONLY) {
+  if constexpr (MODE != TV_ONLY && kOwn) {
 #pragma unroll
     for (int j = 0; j < RY; ++j) {
       if constexpr (kYbInLds) {
@@ -413,9 +407,6 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
       }
     }
   }
-  if constexpr (ENERGY)
-    for (int i = threadIdx.x; i < kEnergyFrames * BY * EnergySlots<D>::kPerWave; i += blockDim.x)
-      red[i] = 0.f;
   float err = 0.f;
 
   // Frame t+1's x and Phi are requested before frame t's TV so that their
@@ -433,8 +424,8 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
     if constexpr (MODE != TV_ONLY) dma_rows<RY>(phit, N, dma_ph, off0, W, lp.lane);
     if (!from_y) dma_rows<RY>(xt, N, dma_x, off0, W, lp.lane);
   } else {
-    if constexpr (MODE != TV_ONLY) load_plane<RY, INSIDE>(phit, nph, lp, off0, H, W);
-    if (!from_y) load_plane<RY, INSIDE>(xt, nx, lp, off0, H, W);
+    if constexpr (MODE != TV_ONLY) load_plane<RY, COVER>(phit, nph, lp, off0, H, W);
+    if (!from_y) load_plane<RY, COVER>(xt, nx, lp, off0, H, W);
   }
 
   float* xo = a.x_out + size_t(t_lo) * N;
@@ -446,7 +437,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
   // Every lane reads back only the LDS slots it wrote itself (the one-barrier
   // engine synchronises before it reads a neighbour's rows).
   float2* const img = sh.img + sl0;
-  const bool owns_any = tp.own_r != 0;  // wave-uniform: halo waves own nothing
+  const bool owns_any = kOwn && tp.own_r != 0;  // wave-uniform
   for (int t = 0; t < T; ++t) {
     float ph[RY][2];
     if constexpr (kDma) {
@@ -505,9 +496,9 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
           if (r < lo || r >= hi) continue;
           if (r < RY) {
             if constexpr (MODE != TV_ONLY)
-              load_row<RY, INSIDE>(phit + nstep, nph, lp, off0, H, W, r);
+              load_row<RY, COVER>(phit + nstep, nph, lp, off0, H, W, r);
           } else if (!from_y) {
-            load_row<RY, INSIDE>(xt + nstep, nx, lp, off0, H, W, r - RY);
+            load_row<RY, COVER>(xt + nstep, nx, lp, off0, H, W, r - RY);
           }
         }
       }
@@ -515,14 +506,16 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
 
     float out[RY][2];
     float acc[NH * 8];
-    if constexpr (X1) {
-      tv_run_x1<D, RY, BY, NH, !INSIDE>(img, out, D, lds, lp, em, a.weight, a.tw, acc, ENERGY,
+    if constexpr (!kOwn) {
+      tv_run_halo<D, RY, BY, EDGE, STRIP>(img, lds, lp, em, a.tw, prefetch);
+    } else if constexpr (X1) {
+      tv_run_x1<D, RY, BY, NH, EDGE>(img, out, D, lds, lp, em, a.weight, a.tw, acc, ENERGY,
                                         prefetch);
     } else
-      tv_run_from_zero<D, RY, BY, NH, !INSIDE>(img, out, D, lds, lp, em, a.weight, a.tw, acc,
+      tv_run_from_zero<D, RY, BY, NH, EDGE>(img, out, D, lds, lp, em, a.weight, a.tw, acc,
                                                ENERGY, prefetch);
 
-    if (owns_any) {
+    if constexpr (kOwn) if (owns_any) {
       float bv[RY][2];
 #pragma unroll
       for (int j = 0; j < RY; ++j) {
@@ -564,8 +557,8 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
       if (tp.own_c[0]) {
         unsigned base = unsigned(off0) * 4u;
         compute_here(base);
-        // In an interior tile of one-strip waves (MR = 1) a wave that owns
-        // any row owns all of them: strips 1 .. BY-2 are the tile interior.
+        // An inside strip (MR = 1) that owns any row owns all of them: strips
+        // 1 .. BY-2 are the tile interior.
         constexpr bool kAllRows = INSIDE && MR == 1;
         store_owned<D, BY, MR, INSIDE, RY, kAllRows>(xo, N, W, tp, base, out);
         if constexpr (MODE == ADMM) {
@@ -573,7 +566,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
         }
       }
     }
-    if constexpr (kYbInLds && MODE != TV_ONLY) {
+    if constexpr (kYbInLds && MODE != TV_ONLY && kOwn) {
       if (owns_any && (t % kYbBlock == kYbBlock - 1 || t == T - 1)) {  // wave-uniform
 #pragma unroll
         for (int j = 0; j < RY; ++j)
@@ -586,7 +579,9 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
     }
     if constexpr (ENERGY) {
       const int tb = t % kEnergyFrames;
-      energy_add<D, BY, MR, NH>(acc, tp.lane_owner, red + tb * BY * EnergySlots<D>::kPerWave, lp);
+      if constexpr (kOwn)
+        energy_add<D, BY, MR, NH>(acc, tp.lane_owner, red + tb * BY * EnergySlots<D>::kPerWave,
+                                  lp);
       if (es && (tb == kEnergyFrames - 1 || t == T - 1))  // workgroup-uniform
         energy_store<D, BY>(red, tb + 1, es - size_t(tb) * D * es_stride, es_stride, tile_id);
     }
@@ -598,7 +593,7 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
     if constexpr (MODE == ADMM) bt += (bt ? N : 0);
   }
 
-  if constexpr (MODE != TV_ONLY) {
+  if constexpr (MODE != TV_ONLY && kOwn) {
 #pragma unroll
     for (int j = 0; j < RY; ++j) {
       if (!((tp.own_r >> j) & 1u)) continue;
@@ -618,6 +613,93 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
     }
   }
   if constexpr (IQA) commit_err<BY>(err, a.err, red64, lp.w, lp.lane);
+}
+
+// A strip with no row in the image: the rows that it publishes are zero, and
+// it owns nothing.  It meets the barriers of the tile's other strips.
+template <int D, int BY, int MR, bool IQA, bool ENERGY>
+__device__ __forceinline__ void fused_strip_empty(const FusedArgs& a, int tile,
+                                                  FusedLds<D, BY, MR>& sh, int part, int strip) {
+  const int lane = threadIdx.x & 63;
+  reinterpret_cast<float2*>(sh.eng.xo)[strip * 64 + lane] = make_float2(0.f, 0.f);
+  reinterpret_cast<float2*>(sh.eng.xp)[(strip + 1) * 64 + lane] = make_float2(0.f, 0.f);
+  const int nparts = a.fsplit > 1 ? a.fsplit : 1;
+  const int t_lo = (a.T * part) / nparts, T = (a.T * (part + 1)) / nparts - t_lo;
+  for (int t = 0; t < T; ++t) {
+    for (int u = 0; u < 2 * D; ++u) __syncthreads();  // tv_run_from_zero
+    if constexpr (ENERGY) {
+      const int tb = t % kEnergyFrames;
+      if (a.eslot && (tb == kEnergyFrames - 1 || t == T - 1))
+        energy_store<D, BY>(sh.red, tb + 1,
+                            a.eslot + size_t(t_lo + t - tb) * D * a.eslot_stride, a.eslot_stride,
+                            tile);
+    }
+  }
+  if constexpr (IQA) commit_err<BY>(0.f, a.err, sh.red64, strip, lane);
+}
+
+// One tile of one fused outer iteration (the body of k_fused and of the
+// batched persistent kernel).  Each wave runs the body of its strip, chosen by
+// where the strip lies; all bodies meet the same barriers.
+//  * A strip inside the image needs no masks; one that also ends at the last
+//    column masks one gradient of its four.  Only strips that hold rows or
+//    columns outside the image, or its last row, mask everything.
+//  * The halo strips of such tiles update the rows that the result depends on,
+//    and strips beyond the image nothing.
+// A launch ends with its slowest tiles.  With masks and per-pixel loads chosen
+// per tile, a border tile of 256x256x8 (15 of 33 are) held its first frame
+// 1.2 us later than an interior one and took 3.4 us over it instead of 2.8.
+// Per strip, the launch takes 11.7 us instead of 12.8 there, and 295 us
+// instead of 316 at 2048x2048x20; of the latter the halo strips' rows are 4 us.
+// Without STRIPS (the launches split by tile class) only the masks are chosen.
+template <int D, int BY, int MR, int MODE, bool IQA, bool X1 = false, bool DMA = false,
+          bool ENERGY = true, bool STRIPS = true>
+__device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
+                                           FusedLds<D, BY, MR, X1, DMA>& sh, int part = 0) {
+  using G = TileGeom<D, BY, MR>;
+  if constexpr (!X1) sh.eng.zero_edges();
+  if constexpr (ENERGY)
+    for (int i = threadIdx.x; i < kEnergyFrames * BY * EnergySlots<D>::kPerWave; i += blockDim.x)
+      sh.red[i] = 0.f;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
+  const ColPlace cp = col_place(tx, a.tiles_x, a.W, G::LW, G::HC, G::OX);
+  const int row0 = ty * G::OY - D + w * G::RY, row1 = row0 + G::RY;
+  const bool cols = cp.c0 >= 0 && cp.c0 + G::LW <= a.W;
+  // (The gradient of the last strip's last row is not used.)
+  const bool inside = cols && row0 >= 0 && row1 <= a.H - (w == BY - 1 ? 0 : 1);
+  auto run = [&](auto cover, auto edge, auto kind) __attribute__((always_inline)) {
+    fused_strip<D, BY, MR, MODE, Cover(decltype(cover)::value), Edge(decltype(edge)::value), IQA,
+                X1, DMA, ENERGY, StripKind(decltype(kind)::value)>(a, tile, sh, part, w);
+  };
+  using std::integral_constant;
+  constexpr integral_constant<int, COVER_NONE> some{};
+  constexpr integral_constant<int, COVER_COLS> columns{};
+  constexpr integral_constant<int, COVER_ALL> all{};
+  constexpr integral_constant<int, EDGE_NONE> none{};
+  constexpr integral_constant<int, EDGE_RIGHT> right{};
+  constexpr integral_constant<int, EDGE_ANY> any{};
+  constexpr integral_constant<int, STRIP_OWN> own{};
+  constexpr bool kHaloBodies = D <= 4;  // (deeper ones would spill a register)
+  if constexpr (!STRIPS || X1 || DMA || MR != 1) {
+    if (inside && !cp.edge_right) run(all, none, own);
+    else run(some, any, own);
+  } else if (row1 <= 0 || row0 >= a.H) {
+    fused_strip_empty<D, BY, MR, IQA, ENERGY>(a, tile, sh, part, w);
+  } else if (inside && !cp.edge_right) {
+    if (kHaloBodies && w == 0)
+      run(all, none, integral_constant<int, kHaloBodies ? STRIP_TOP : STRIP_OWN>{});
+    else if (kHaloBodies && w == BY - 1)
+      run(all, none, integral_constant<int, kHaloBodies ? STRIP_BOTTOM : STRIP_OWN>{});
+    else
+      run(all, none, own);
+  } else if (inside) {
+    run(all, right, own);
+  } else if (cols) {
+    run(columns, any, own);
+  } else {
+    run(some, any, own);
+  }
 }
 
 // Sum of the frame parts' yb and the residual epilogue (fsplit > 1): the
@@ -651,10 +733,9 @@ __host__ __device__ inline bool tile_inside(int tile, int tiles_x, int H, int W)
          !cp.edge_right;
 }
 
-// One launch covers interior and border tiles; the two bodies are separate
-// instantiations (the interior one has no masks or bounds checks).  PART
-// restricts a launch to one class (1: interior, 2: border; 0: both), so that
-// the interior kernel is allocated registers for its own body only.  With the
+// One launch covers interior and border tiles.  PART restricts a launch to
+// one class (1: interior, 2: border; 0: both), so that the interior kernel is
+// allocated registers for its own body only.  With the
 // per-iteration error (IQA) the 8-wave kernel is held to 128 VGPRs, the limit
 // for two workgroups per CU (it would take 130-133; with one workgroup per CU
 // a 2048x2048x20 solve takes 48 ms instead of 32).
@@ -669,16 +750,8 @@ __attribute__((amdgpu_waves_per_eu(BY == 8 && D <= 4 && IQA ? 4 : 1))) k_fused(F
   if (item >= a.ntiles) return;
   const int nparts = a.fsplit > 1 ? a.fsplit : 1;
   const int tile = item / nparts, part = item - tile * nparts;
-  const bool inside = tile_inside<D, BY, MR>(tile, a.tiles_x, a.H, a.W);
-  if constexpr (PART != 2) {
-    if (inside) {
-      fused_tile<D, BY, MR, MODE, true, IQA, X1, DMA>(a, tile, sh, part);
-      return;
-    }
-  }
-  if constexpr (PART != 1) {
-    if (!inside) fused_tile<D, BY, MR, MODE, false, IQA, X1>(a, tile, sh, part);
-  }
+  if (PART != 0 && tile_inside<D, BY, MR>(tile, a.tiles_x, a.H, a.W) != (PART == 1)) return;
+  fused_tile<D, BY, MR, MODE, IQA, X1, DMA, true, PART == 0>(a, tile, sh, part);
 }
 
 // Early-exit decision of one frame (workgroup blockIdx.x; NT threads): the
@@ -778,6 +851,7 @@ __device__ __forceinline__ void fused_fix_tile(const FusedArgs& a, int tile, Fix
   constexpr int RY = G::RY;
   constexpr int NH = MR;
   constexpr bool kTvOnly = MODE == TV_ONLY;
+  constexpr int kCover = INSIDE ? COVER_ALL : COVER_NONE;
   TileLds<BY>& lds = sh.eng;
   lds.zero_edges();
   double* const red64 = sh.red64;
@@ -793,10 +867,10 @@ __device__ __forceinline__ void fused_fix_tile(const FusedArgs& a, int tile, Fix
   // q = lambda*r (or y + lambda*r when X_0 = At(y)), as in the main pass.
   float q[RY][2] = {};
   if constexpr (!kTvOnly) {
-    load_plane<RY, INSIDE>(a.r_in, q, lp, off0, H, W);
+    load_plane<RY, kCover>(a.r_in, q, lp, off0, H, W);
     if (from_y) {
       float yv[RY][2];
-      load_plane<RY, INSIDE>(a.y, yv, lp, off0, H, W);
+      load_plane<RY, kCover>(a.y, yv, lp, off0, H, W);
 #pragma unroll
       for (int j = 0; j < RY; ++j)
 #pragma unroll
@@ -826,8 +900,8 @@ __device__ __forceinline__ void fused_fix_tile(const FusedArgs& a, int tile, Fix
   int t = next_stopped(0);
   float nph[RY][2] = {}, nx[RY][2] = {};
   if (t < T) {
-    if constexpr (!kTvOnly) load_plane<RY, INSIDE>(a.phi + size_t(t) * N, nph, lp, off0, H, W);
-    if (!from_y) load_plane<RY, INSIDE>(a.x_in + size_t(t) * N, nx, lp, off0, H, W);
+    if constexpr (!kTvOnly) load_plane<RY, kCover>(a.phi + size_t(t) * N, nph, lp, off0, H, W);
+    if (!from_y) load_plane<RY, kCover>(a.x_in + size_t(t) * N, nx, lp, off0, H, W);
   }
   // Every lane reads back only the LDS slots it wrote itself.
   float2* const simg = sh.img + lp.w * RY * 64 + lp.lane;
@@ -858,12 +932,12 @@ __device__ __forceinline__ void fused_fix_tile(const FusedArgs& a, int tile, Fix
       for (int r = 0; r < total; ++r) {
         if (r < lo || r >= hi) continue;
         if (r < RY) {
-          if constexpr (!kTvOnly) load_row<RY, INSIDE>(xo, xold, lp, off0, H, W, r);
+          if constexpr (!kTvOnly) load_row<RY, kCover>(xo, xold, lp, off0, H, W, r);
         } else if (r < 2 * RY) {
           if constexpr (!kTvOnly)
-            if (tn < T) load_row<RY, INSIDE>(nphi, nph, lp, off0, H, W, r - RY);
+            if (tn < T) load_row<RY, kCover>(nphi, nph, lp, off0, H, W, r - RY);
         } else if (!from_y && tn < T) {
-          load_row<RY, INSIDE>(nxin, nx, lp, off0, H, W, r - 2 * RY);
+          load_row<RY, kCover>(nxin, nx, lp, off0, H, W, r - 2 * RY);
         }
       }
     };

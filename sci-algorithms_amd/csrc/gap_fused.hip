@@ -443,10 +443,7 @@ __global__ void __launch_bounds__(64 * BY) k_fused_samples(FusedArgs a, SampleSt
   const int nparts = a.fsplit > 1 ? a.fsplit : 1;
   const int tile = rest / nparts, part = rest - tile * nparts;
   select_sample(a, st, b);
-  if (tile_inside<D, BY, 1>(tile, a.tiles_x, a.H, a.W))
-    fused_tile<D, BY, 1, GAP_ACC, true, false, false, false, false>(a, tile, sh, part);
-  else
-    fused_tile<D, BY, 1, GAP_ACC, false, false, false, false, false>(a, tile, sh, part);
+  fused_tile<D, BY, 1, GAP_ACC, false, false, false, false>(a, tile, sh, part);
 }
 
 __global__ void __launch_bounds__(256) k_part_epilogue_samples(FusedArgs a, SampleStrides st) {

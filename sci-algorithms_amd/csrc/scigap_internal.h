@@ -1,6 +1,7 @@
 // Internal helpers shared by the scigap HIP sources (not part of the C ABI).
 #pragma once
 
+#include <utility>
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -91,6 +92,17 @@ __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcp
 // every term of the sum live until then.
 __device__ __forceinline__ void compute_here(float& v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void compute_here(unsigned& v) { asm volatile("" : "+v"(v)); }
+
+// f(0), ..., f(N-1) with compile-time indices: per-row register arrays are
+// then registers from the start, not only after a loop has been unrolled.
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
 
 // Per-pixel sums over the frames (A x = sum_t Phi_t x_t and its corrections)
 // are accumulated in fp64 from the exact products of the fp32 factors and

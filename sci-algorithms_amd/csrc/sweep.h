@@ -37,17 +37,6 @@ extern "C" __device__ void raw_buffer_store_f2(f2 v, __amdgpu_buffer_rsrc_t rsrc
                                                int soffset, int aux)
     __asm("llvm.amdgcn.raw.ptr.buffer.store.v2f32");
 
-// f(0), ..., f(N-1) with compile-time indices: the strips' row arrays must be
-// registers from the start, not only after a loop of this size is unrolled.
-template <class F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 // A wave-uniform float as a scalar register: an FMA that reads two vector
 // registers and a scalar issues at the rate of an add, one that reads three
 // vector registers takes 4 cycles instead of 2.6 (two or more waves a SIMD).

@@ -237,13 +237,13 @@ __device__ __forceinline__ void bwd_tile(const BwdArgs& a, int tile, int t, BwdL
   float vr[RY][2], xb[RY][2];
   {
     float xv[RY][2], ph[RY][2];
-    load_plane<RY, INSIDE>(a.r, vr, lp, off0, H, W);
-    load_plane<RY, INSIDE>(a.x + size_t(t) * N, xv, lp, off0, H, W);
-    load_plane<RY, INSIDE>(a.phi + size_t(t) * N, ph, lp, off0, H, W);
-    load_plane<RY, INSIDE>(a.xbar + size_t(t) * N, xb, lp, off0, H, W);
+    load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(a.r, vr, lp, off0, H, W);
+    load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(a.x + size_t(t) * N, xv, lp, off0, H, W);
+    load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(a.phi + size_t(t) * N, ph, lp, off0, H, W);
+    load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(a.xbar + size_t(t) * N, xb, lp, off0, H, W);
     if (a.ybb) {
       float yb[RY][2];
-      load_plane<RY, INSIDE>(a.ybb, yb, lp, off0, H, W);
+      load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(a.ybb, yb, lp, off0, H, W);
 #pragma unroll
       for (int j = 0; j < RY; ++j)
 #pragma unroll

@@ -110,11 +110,11 @@ __device__ __forceinline__ void chunk_tile(const ChunkArgs& a, int tile, ChunkLd
     const int nup = REPAIR ? a.fix[t] : (a.stop[t] < 0 ? a.nup : -1);  // uniform
     if (nup >= 0) {
       float v[RY][2], p0[RY][2], p1[RY][2];
-      load_plane<RY, INSIDE>(a.img + size_t(t) * N, v, lp, off0, H, W);
+      load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(a.img + size_t(t) * N, v, lp, off0, H, W);
       if (a.p_in) {
         const float* pt = a.p_in + size_t(t) * 2 * N;
-        load_plane<RY, INSIDE>(pt, p0, lp, off0, H, W);
-        load_plane<RY, INSIDE>(pt + N, p1, lp, off0, H, W);
+        load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(pt, p0, lp, off0, H, W);
+        load_plane<RY, INSIDE ? COVER_ALL : COVER_NONE>(pt + N, p1, lp, off0, H, W);
       } else {
 #pragma unroll
         for (int j = 0; j < RY; ++j) p0[j][0] = p0[j][1] = p1[j][0] = p1[j][1] = 0.f;

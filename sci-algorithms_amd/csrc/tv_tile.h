@@ -88,6 +88,7 @@ struct EdgeMasks {
   unsigned rowin = 0;   // bit j: 0 <= row0+j < H     (horizontal difference)
   float colin[2];       // 0 <= col+k < W             (vertical difference)
   float colok1[2];      // 0 <= col+k < W-1           (horizontal difference)
+  __device__ void init_right(const LanePos& lp, int W) { colok1[1] = lp.col + 1 < W - 1 ? 1.f : 0.f; }
   template <int RY>
   __device__ void init(const LanePos& lp, int H, int W) {
     rowok0 = rowin = 0;
@@ -111,6 +112,54 @@ struct EdgeMasks {
 // [0, RY/2) and half 1 rows [RY/2, RY) of the lane's strip (needed when a
 // wave holds both halo and interior rows); with NH = 1 one sum per update.
 
+// dq of row j at this lane's two columns; `up` is row j-1 of q0.
+__device__ __forceinline__ void div_row(float up0, float up1, const float (&p0)[2],
+                                        const float (&p1)[2], float& d0, float& d1) {
+  const float left0 = from_prev_lane(p1[1]);
+  d0 = (up0 - p0[0]) + (left0 - p1[0]);
+  d1 = (up1 - p0[1]) + (p1[0] - p1[1]);
+}
+
+// Masks of a strip's dual updates.
+enum Edge {
+  EDGE_NONE = 0,   // no gradient to mask
+  EDGE_ANY = 1,    // rows or columns outside the image, or its last row
+  EDGE_RIGHT = 2,  // ends at the image's last column, otherwise as EDGE_NONE
+};
+
+// Dual update of row j from its own `out` row and the row below (dn); ZERO:
+// q = 0 before it.  Returns |g| of the two columns.
+template <int EDGE, bool ZERO>
+__device__ __forceinline__ float2 dual_row(const float (&out)[2], float dn0, float dn1,
+                                           float (&p0)[2], float (&p1)[2], const EdgeMasks& em,
+                                           int j, float tw) {
+  const float right1 = from_next_lane(out[0]);
+  float g00 = dn0 - out[0];
+  float g01 = dn1 - out[1];
+  float g10 = out[1] - out[0];
+  float g11 = right1 - out[1];
+  if constexpr (EDGE == EDGE_RIGHT) g11 *= em.colok1[1];
+  if constexpr (EDGE == EDGE_ANY) {
+    const bool v_ok = (em.rowok0 >> j) & 1u, h_ok = (em.rowin >> j) & 1u;
+    g00 = v_ok ? g00 * em.colin[0] : 0.f;
+    g01 = v_ok ? g01 * em.colin[1] : 0.f;
+    g10 = h_ok ? g10 * em.colok1[0] : 0.f;
+    g11 = h_ok ? g11 * em.colok1[1] : 0.f;
+  }
+  const float n0 = fast_sqrt(fmaf(g00, g00, g10 * g10));
+  const float n1 = fast_sqrt(fmaf(g01, g01, g11 * g11));
+  const float i0 = fast_rcp(fmaf(tw, n0, 1.f));
+  const float i1 = fast_rcp(fmaf(tw, n1, 1.f));
+  p0[0] = (ZERO ? g00 : p0[0] + g00) * i0;
+  p1[0] = (ZERO ? g10 : p1[0] + g10) * i0;
+  p0[1] = (ZERO ? g01 : p0[1] + g01) * i1;
+  p1[1] = (ZERO ? g11 : p1[1] + g11) * i1;
+  // Materialise the new dual values here; otherwise the compiler folds the
+  // multiply by 1/den into the next divergence and keeps both factors live.
+  asm("" : "+v"(p0[0]), "+v"(p1[0]), "+v"(p0[1]), "+v"(p1[1]));
+  return make_float2(n0, n1);
+}
+
 // out = img + d(p), with img read from LDS (row j at img[j*64]); adds sum d^2
 // of each strip half h to dacc[h*8] when dacc is non-null.
 template <int RY, int BY, int NH>
@@ -133,11 +182,8 @@ __device__ __forceinline__ void tv_div(const float2* img, float (&out)[RY][2],
 #pragma unroll
   for (int jj = 0; jj < RY; ++jj) {
     const int j = jj + 1 < RY ? jj + 1 : 0;
-    float up0 = j > 0 ? p0[j - 1][0] : above.x;
-    float up1 = j > 0 ? p0[j - 1][1] : above.y;
-    float left0 = from_prev_lane(p1[j][1]);
-    d0[j] = (up0 - p0[j][0]) + (left0 - p1[j][0]);
-    d1[j] = (up1 - p0[j][1]) + (p1[j][0] - p1[j][1]);
+    div_row(j > 0 ? p0[j - 1][0] : above.x, j > 0 ? p0[j - 1][1] : above.y, p0[j], p1[j], d0[j],
+            d1[j]);
     out[j][0] = fmaf(-0.25f, d0[j], im[j].x);
     out[j][1] = fmaf(-0.25f, d1[j], im[j].y);
   }
@@ -159,7 +205,7 @@ __device__ __forceinline__ void tv_div(const float2* img, float (&out)[RY][2],
 // One dual update q <- (q + g)/(1 + tw |g|) from the current `out` (ZERO:
 // q = 0 before it, the first update); adds weight*sum|g| of each strip half h
 // to gacc[h*8] when gacc is non-null.
-template <int RY, int BY, int NH, bool EDGE, bool ZERO = false>
+template <int RY, int BY, int NH, int EDGE, bool ZERO = false>
 __device__ __forceinline__ void tv_grad(const float (&out)[RY][2], float (&p0)[RY][2],
                                         float (&p1)[RY][2], TileLds<BY>& lds, const LanePos& lp,
                                         const EdgeMasks& em, float weight, float tw, float* gacc) {
@@ -172,32 +218,10 @@ __device__ __forceinline__ void tv_grad(const float (&out)[RY][2], float (&p0)[R
   for (int j = 0; j < RY; ++j) {
     float dn0 = j + 1 < RY ? out[j + 1][0] : below.x;
     float dn1 = j + 1 < RY ? out[j + 1][1] : below.y;
-    float right1 = from_next_lane(out[j][0]);
-    float g00 = dn0 - out[j][0];
-    float g01 = dn1 - out[j][1];
-    float g10 = out[j][1] - out[j][0];
-    float g11 = right1 - out[j][1];
-    if constexpr (EDGE) {
-      const bool v_ok = (em.rowok0 >> j) & 1u, h_ok = (em.rowin >> j) & 1u;
-      g00 = v_ok ? g00 * em.colin[0] : 0.f;
-      g01 = v_ok ? g01 * em.colin[1] : 0.f;
-      g10 = h_ok ? g10 * em.colok1[0] : 0.f;
-      g11 = h_ok ? g11 * em.colok1[1] : 0.f;
-    }
-    float n0 = fast_sqrt(fmaf(g00, g00, g10 * g10));
-    float n1 = fast_sqrt(fmaf(g01, g01, g11 * g11));
+    const float2 n = dual_row<EDGE, ZERO>(out[j], dn0, dn1, p0[j], p1[j], em, j, tw);
     const int h = (NH == 2 && j >= RY / 2) ? 1 : 0;
     // The first row of a half assigns (0 + x would be an instruction).
-    s[h] = j == h * (RY / 2) ? n0 + n1 : s[h] + (n0 + n1);
-    float i0 = fast_rcp(fmaf(tw, n0, 1.f));
-    float i1 = fast_rcp(fmaf(tw, n1, 1.f));
-    p0[j][0] = (ZERO ? g00 : p0[j][0] + g00) * i0;
-    p1[j][0] = (ZERO ? g10 : p1[j][0] + g10) * i0;
-    p0[j][1] = (ZERO ? g01 : p0[j][1] + g01) * i1;
-    p1[j][1] = (ZERO ? g11 : p1[j][1] + g11) * i1;
-    // Materialise the new dual values here; otherwise the compiler folds the
-    // multiply by 1/den into the next divergence and keeps both factors live.
-    asm("" : "+v"(p0[j][0]), "+v"(p1[j][0]), "+v"(p0[j][1]), "+v"(p1[j][1]));
+    s[h] = j == h * (RY / 2) ? n.x + n.y : s[h] + (n.x + n.y);
   }
   if (gacc)
 #pragma unroll
@@ -219,7 +243,7 @@ struct NoHook {
   __device__ void operator()(int) const {}
 };
 
-template <int D, int RY, int BY, int NH, bool EDGE, class Hook = NoHook>
+template <int D, int RY, int BY, int NH, int EDGE, class Hook = NoHook>
 __device__ __forceinline__ void tv_run_from_zero(const float2* img, float (&out)[RY][2], int nup,
                                                  TileLds<BY>& lds, const LanePos& lp,
                                                  const EdgeMasks& em, float weight, float tw,
@@ -255,6 +279,65 @@ __device__ __forceinline__ void tv_run_from_zero(const float2* img, float (&out)
   }
 }
 
+// Rows of a tile's halo strips (MR = 1, so that wave 0 and the last wave hold
+// halo rows only).  After update u (0-based) the tile's result depends on the
+// rows [u, RY) of the top strip and [0, RY-2-u] of the bottom one; their `out`
+// after the last update is not needed at all, nor are their energies.  Of the
+// 2*RY*D row updates of the two strips D*D remain, 12.5% less of an 8-wave
+// tile with D = 4.  Barriers and published rows are those of tv_run_from_zero,
+// which the other waves run at the same time, and so are the values of every
+// row that is updated.
+enum StripKind { STRIP_OWN = 0, STRIP_TOP = 1, STRIP_BOTTOM = 2 };
+
+template <int D, int RY, int BY, int EDGE, StripKind STRIP, class Hook>
+__device__ __forceinline__ void tv_run_halo(const float2* img, TileLds<BY>& lds,
+                                            const LanePos& lp, const EdgeMasks& em, float tw,
+                                            const Hook& hook) {
+  static_assert(RY == D && STRIP != STRIP_OWN, "halo strips have D rows");
+  constexpr bool kTop = STRIP == STRIP_TOP;
+  float2* const xo = reinterpret_cast<float2*>(lds.xo);
+  float2* const xp = reinterpret_cast<float2*>(lds.xp);
+  float out[RY][2], p0[RY][2], p1[RY][2];
+#pragma unroll
+  for (int j = 0; j < RY; ++j) {
+    const float2 im = img[j * 64];
+    out[j][0] = im.x;
+    out[j][1] = im.y;
+  }
+  static_for<D>([&](auto uc) __attribute__((always_inline)) {
+    constexpr int u = decltype(uc)::value;
+    constexpr int glo = kTop ? u : 0, ghi = kTop ? RY - 1 : RY - 2 - u;          // dual rows
+    constexpr int dlo = kTop ? u + 1 : 0;                                        // out rows
+    constexpr int dhi = u + 1 == D ? -1 : (kTop ? RY - 1 : RY - 2 - u);
+    if constexpr (!kTop) xo[lp.w * 64 + lp.lane] = make_float2(out[0][0], out[0][1]);
+    __syncthreads();
+    float2 below = make_float2(0.f, 0.f);
+    if constexpr (kTop) below = xo[(lp.w + 1) * 64 + lp.lane];
+#pragma unroll
+    for (int j = glo; j <= ghi; ++j)
+      dual_row<EDGE, u == 0>(out[j], j + 1 < RY ? out[j + 1 < RY ? j + 1 : 0][0] : below.x,
+                             j + 1 < RY ? out[j + 1 < RY ? j + 1 : 0][1] : below.y, p0[j], p1[j],
+                             em, j, tw);
+    hook(u);
+    if constexpr (kTop) xp[(lp.w + 1) * 64 + lp.lane] = make_float2(p0[RY - 1][0], p0[RY - 1][1]);
+    float2 im[RY];
+#pragma unroll
+    for (int j = dlo; j <= dhi; ++j) im[j] = img[j * 64];
+    __syncthreads();
+    float2 above = make_float2(0.f, 0.f);
+    if constexpr (!kTop && dhi >= 0) above = xp[lp.w * 64 + lp.lane];
+#pragma unroll
+    for (int jj = dlo; jj <= dhi; ++jj) {
+      const int j = kTop ? jj : dhi - jj;  // row 0, which waits for `above`, last
+      float d0, d1;
+      div_row(j > 0 ? p0[j > 0 ? j - 1 : 0][0] : above.x, j > 0 ? p0[j > 0 ? j - 1 : 0][1] : above.y,
+              p0[j], p1[j], d0, d1);
+      out[j][0] = fmaf(-0.25f, d0, im[j].x);
+      out[j][1] = fmaf(-0.25f, d1, im[j].y);
+    }
+  });
+}
+
 // One-barrier variant of the engine.  Each update publishes, per wave, the
 // new p0 of its last row (the wave below needs it for its first divergence
 // row) and the new p0, p1 of its first row, from which the wave above forms
@@ -271,7 +354,7 @@ struct TileLdsX1 {
 
 // Dual update from `out` with the next wave's first `out` row in `below`
 // (no LDS traffic); adds weight*sum|g| per strip half to gacc[h*8].
-template <int RY, int NH, bool EDGE, bool ZERO = false>
+template <int RY, int NH, int EDGE, bool ZERO = false>
 __device__ __forceinline__ void tv_grad_regs(const float (&out)[RY][2], float2 below,
                                              float (&p0)[RY][2], float (&p1)[RY][2],
                                              const EdgeMasks& em, float weight, float tw,
@@ -281,30 +364,10 @@ __device__ __forceinline__ void tv_grad_regs(const float (&out)[RY][2], float2 b
   for (int j = 0; j < RY; ++j) {
     float dn0 = j + 1 < RY ? out[j + 1][0] : below.x;
     float dn1 = j + 1 < RY ? out[j + 1][1] : below.y;
-    float right1 = from_next_lane(out[j][0]);
-    float g00 = dn0 - out[j][0];
-    float g01 = dn1 - out[j][1];
-    float g10 = out[j][1] - out[j][0];
-    float g11 = right1 - out[j][1];
-    if constexpr (EDGE) {
-      const bool v_ok = (em.rowok0 >> j) & 1u, h_ok = (em.rowin >> j) & 1u;
-      g00 = v_ok ? g00 * em.colin[0] : 0.f;
-      g01 = v_ok ? g01 * em.colin[1] : 0.f;
-      g10 = h_ok ? g10 * em.colok1[0] : 0.f;
-      g11 = h_ok ? g11 * em.colok1[1] : 0.f;
-    }
-    float n0 = fast_sqrt(fmaf(g00, g00, g10 * g10));
-    float n1 = fast_sqrt(fmaf(g01, g01, g11 * g11));
+    const float2 n = dual_row<EDGE, ZERO>(out[j], dn0, dn1, p0[j], p1[j], em, j, tw);
     const int h = (NH == 2 && j >= RY / 2) ? 1 : 0;
     // The first row of a half assigns (0 + x would be an instruction).
-    s[h] = j == h * (RY / 2) ? n0 + n1 : s[h] + (n0 + n1);
-    float i0 = fast_rcp(fmaf(tw, n0, 1.f));
-    float i1 = fast_rcp(fmaf(tw, n1, 1.f));
-    p0[j][0] = (ZERO ? g00 : p0[j][0] + g00) * i0;
-    p1[j][0] = (ZERO ? g10 : p1[j][0] + g10) * i0;
-    p0[j][1] = (ZERO ? g01 : p0[j][1] + g01) * i1;
-    p1[j][1] = (ZERO ? g11 : p1[j][1] + g11) * i1;
-    asm("" : "+v"(p0[j][0]), "+v"(p1[j][0]), "+v"(p0[j][1]), "+v"(p1[j][1]));
+    s[h] = j == h * (RY / 2) ? n.x + n.y : s[h] + (n.x + n.y);
   }
   if (gacc)
 #pragma unroll
@@ -322,11 +385,8 @@ __device__ __forceinline__ void tv_div_regs(const float2* img, float (&out)[RY][
   float s[NH] = {};
 #pragma unroll
   for (int j = 0; j < RY; ++j) {
-    float up0 = j > 0 ? p0[j - 1][0] : above.x;
-    float up1 = j > 0 ? p0[j - 1][1] : above.y;
-    float left0 = from_prev_lane(p1[j][1]);
-    float d0 = (up0 - p0[j][0]) + (left0 - p1[j][0]);
-    float d1 = (up1 - p0[j][1]) + (p1[j][0] - p1[j][1]);
+    float d0, d1;
+    div_row(j > 0 ? p0[j - 1][0] : above.x, j > 0 ? p0[j - 1][1] : above.y, p0[j], p1[j], d0, d1);
     const float2 im = img[j * 64];
     out[j][0] = fmaf(-0.25f, d0, im.x);
     out[j][1] = fmaf(-0.25f, d1, im.y);
@@ -345,7 +405,7 @@ __device__ __forceinline__ void tv_div_regs(const float2* img, float (&out)[RY][
 // tv_run_from_zero with one barrier per update (plus one at entry, after
 // which the img rows of the wave below are read).  Same arguments and
 // results, bit for bit; hook(u) runs after the dual step of update u.
-template <int D, int RY, int BY, int NH, bool EDGE, class Hook = NoHook>
+template <int D, int RY, int BY, int NH, int EDGE, class Hook = NoHook>
 __device__ __forceinline__ void tv_run_x1(const float2* img, float (&out)[RY][2], int nup,
                                           TileLdsX1<BY>& lds, const LanePos& lp,
                                           const EdgeMasks& em, float weight, float tw,
