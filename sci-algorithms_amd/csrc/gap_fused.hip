@@ -101,7 +101,6 @@ void launch_kernel(const FusedArgs& a, unsigned grid, hipStream_t s) {
 //      images)
 // The alternatives 2-5 exist for tv_iter_max = 5 (D = 4).  engine 0 is 6.
 constexpr int kDefaultEngine = 6;
-constexpr int kMaxParts = 8;  // frame parts (yb_part planes in the workspace)
 
 // Workgroups of the fused kernel <D, BY, MODE, IQA> resident on the whole
 // device (queried once per instantiation; every device of a process is
