@@ -53,3 +53,18 @@ def test_reverse_sweep_matches_fp64_autograd(gpu, H, W, n):
     assert rel(got["x"], want["x"]) <= 1e-4
     for k in ("mask", "lam", "w"):
         assert rel(got[k], want[k]) <= 1e-3, k
+
+
+@pytest.mark.parametrize("H,W", [(7, 7), (7, 71), (14, 70), (15, 9), (38, 134), (39, 135)])
+def test_ssim_column_walk_matches_oracle(gpu, H, W):
+    """Window centres at the ends of rows of lanes, of a lane's walk and of a
+    workgroup (FP64 in another order: differences of about 49 roundings over the
+    smallest denominator, 9e-4, stay below 1e-11)."""
+    from pnp_sci.device import hwt_to_thw, to_device
+    from pnp_sci.metrics import ssim_frames
+    g = np.random.default_rng(H * W)
+    a = g.random((H, W, 2)).astype(np.float32)
+    b = (a + 0.1 * g.standard_normal(a.shape)).astype(np.float32)
+    got = ssim_frames(hwt_to_thw(to_device(a)), hwt_to_thw(to_device(b)))
+    for t in range(2):
+        assert abs(got[t] - O.compare_ssim(a[..., t], b[..., t])) <= 1e-11
