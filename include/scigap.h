@@ -222,6 +222,19 @@ int scigap_solve(const scigap_params* p,
                  const float* truth, double* sq_err, int* stats,
                  void* workspace, size_t workspace_bytes, void* stream);
 
+/* `solves` reconstructions of one shape and one set of options, sharing the
+ * launches of their iterations: every array holds the solves one after another
+ * (y [solves][H][W], phi [solves][T][H][W], sq_err and stats [solves][iters]).
+ * For the four sub-grids of a Bayer mosaic (pnp_sci_algo.py:95-147), each too
+ * small to fill the GPU.  An explicit tile_rows/engine is used as in
+ * scigap_solve; remembered autotuner choices are not. */
+size_t scigap_solve_many_workspace_bytes(const scigap_params* p, int solves);
+int scigap_solve_many(const scigap_params* p, int solves,
+                      const float* y, const float* phi, const float* phi_sum,
+                      const float* x0, float* x_out,
+                      const float* truth, double* sq_err, int* stats,
+                      void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------- */
 /* Batched solves (mixed-size queue)                                      */
 /* ---------------------------------------------------------------------- */

@@ -49,7 +49,38 @@ struct FusedArgs {
   int fsplit;           // > 1: each tile's frames are split over fsplit workgroups
   float* yb_part;       // [fsplit][H*W] partial yb of each frame part (fsplit > 1)
   int tiles_x, ntiles, per_xcd;
+  // Several solves of one shape in the same launches: the arguments are those
+  // of the first, the others follow at these distances (elements).  The
+  // caller's arrays are packed ([solve][T][H][W] and so on), each solve has a
+  // workspace of its own.  solves <= 1: one solve.
+  int solves;
+  int iters;             // err and stats
+  size_t ws;             // everything in the workspace
+  size_t x_in_b, x_out_b;  // X_k and X_{k+1} (in the workspace or the caller's)
 };
+
+// The arguments of solve b.
+__device__ __forceinline__ void select_solve(FusedArgs& a, int b) {
+  const size_t N = size_t(a.H) * a.W, TN = N * a.T, ws = a.ws * b;
+  a.x_in += a.x_in_b * b;
+  a.x_out += a.x_out_b * b;
+  a.phi += TN * b;
+  a.y += N * b;
+  a.phi_sum += N * b;
+  a.r_in += ws;
+  a.r_out += ws;
+  a.y1_in += ws;
+  a.y1_out += ws;
+  if (a.truth) a.truth += TN * b;
+  a.err += size_t(a.iters) * b;
+  if (a.b) a.b += ws;
+  a.eslot += ws;
+  a.yb += ws;
+  a.stop += ws;
+  a.nexit += ws;
+  if (a.stats) a.stats += size_t(a.iters) * b;
+  a.yb_part += ws;
+}
 
 constexpr int kMaxParts = 8;  // frame parts (yb_part planes in the workspace)
 
@@ -793,10 +824,19 @@ template <int D, int BY, int MR, int MODE, bool IQA, bool X1 = false, int PART =
 __global__ void __launch_bounds__(64 * BY)
 __attribute__((amdgpu_waves_per_eu(BY == 8 && D <= 4 && IQA ? 4 : 1))) k_fused(FusedArgs a) {
   __shared__ FusedLds<D, BY, MR, X1, DMA> sh;
-  // Work item -> (tile, frame part); the parts of a tile are adjacent, so
-  // they run on the same XCD.
-  const int item = tile_of_block(blockIdx.x, a.per_xcd);
-  if (item >= a.ntiles) return;
+  // Work item -> (solve, tile, frame part); the parts of a tile are adjacent,
+  // so they run on the same XCD.
+  int item = tile_of_block(blockIdx.x, a.per_xcd);
+  if constexpr (PART == 0 && !X1 && MODE != TV_ONLY) {
+    const int b = item / a.ntiles;
+    if (item >= a.ntiles) {
+      if (b >= a.solves) return;
+      item -= b * a.ntiles;
+      select_solve(a, b);
+    }
+  } else {
+    if (item >= a.ntiles) return;
+  }
   const int nparts = a.fsplit > 1 ? a.fsplit : 1;
   const int tile = item / nparts, part = item - tile * nparts;
   if (PART != 0 && tile_inside<D, BY, MR>(tile, a.tiles_x, a.H, a.W) != (PART == 1)) return;
@@ -862,6 +902,7 @@ constexpr int kDecideThreads = 1024;
 
 template <int D>
 __global__ void __launch_bounds__(kDecideThreads) k_decide(FusedArgs a) {
+  if (blockIdx.y > 0) select_solve(a, blockIdx.y);
   decide_frame<D, kDecideThreads>(a, blockIdx.x);
 }
 
@@ -872,6 +913,7 @@ __global__ void __launch_bounds__(kDecideThreads) k_decide(FusedArgs a) {
 // launch less per outer iteration where launches dominate (small problems).
 template <int D, int MODE>
 __global__ void __launch_bounds__(kDecideThreads) k_decide_epilogue(FusedArgs a) {
+  if (blockIdx.y > 0) select_solve(a, blockIdx.y);
   if (blockIdx.x < unsigned(a.T)) {  // workgroup-uniform
     decide_frame<D, kDecideThreads>(a, blockIdx.x);
     return;
@@ -1059,6 +1101,8 @@ __global__ void __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(D 
 k_fused_fix(FusedArgs a) {
   __shared__ FixLds<D, BY, MR> sh;
   __shared__ int s_stop[kStopLds];
+  if constexpr (MODE != TV_ONLY)
+    if (blockIdx.y > 0) select_solve(a, blockIdx.y);
   if (*a.nexit == 0) return;  // one scalar load per workgroup
   const int tile = tile_of_block(blockIdx.x, a.per_xcd);
   if (tile >= a.ntiles) return;

@@ -145,17 +145,19 @@ int pick_parts(int tiles, int T, int slots) {
 template <int D, int BY, int MODE, bool IQA, int MR = 1>
 int launch_main(const FusedArgs& a0, hipStream_t s, int engine, int* fold_parts = nullptr) {
   FusedArgs a = a0;
-  const unsigned grid = set_tiles<D, BY, MR>(a);
+  const int solves = std::max(a.solves, 1);
+  set_tiles<D, BY, MR>(a);
   if (engine == 0) engine = kDefaultEngine;
   int parts = 1;
   if (engine == 6 && (MODE == TV_ONLY || a.yb_part)) {
     const int slots = resident_workgroups<D, BY, MODE, IQA, MR>();
-    parts = pick_parts(a.ntiles, a.T, slots);
+    parts = pick_parts(a.ntiles * solves, a.T, slots);
   }
+  a.per_xcd = (a.ntiles * parts * solves + 7) / 8;
+  const unsigned grid = unsigned(a.per_xcd * 8);
   if (parts > 1) {
     a.fsplit = parts;
     a.ntiles *= parts;
-    a.per_xcd = (a.ntiles + 7) / 8;
     ProfScope ps(MODE == TV_ONLY ? "tv_fused" : "fused_iteration", s);
     launch_kernel<D, BY, MODE, IQA, false, 0, false, MR>(a, unsigned(a.per_xcd * 8), s);
     if constexpr (MODE != TV_ONLY) {
@@ -262,7 +264,8 @@ int launch_fused(const FusedArgs& a00, hipStream_t s, int tile_rows, int engine)
   if (!a0.eslot) return fail(SCIGAP_EINVAL, "early exit without energy slots");
   FusedArgs a = a0;
   constexpr int FBY = FixShape<D>::BY;
-  const unsigned grid = set_tiles<D, FBY, MR>(a);
+  const unsigned solves = unsigned(std::max(a.solves, 1));
+  const dim3 grid(set_tiles<D, FBY, MR>(a), solves);
   {
     ProfScope ps("fused_decide", s);
     if (parts > 1) {
@@ -271,7 +274,7 @@ int launch_fused(const FusedArgs& a00, hipStream_t s, int tile_rows, int engine)
       const int64_t N = int64_t(a.H) * a.W;
       const unsigned g =
           unsigned(std::min<int64_t>((N + kDecideThreads - 1) / kDecideThreads, 1024));
-      const unsigned blocks = unsigned(a.T) + g;
+      const dim3 blocks(unsigned(a.T) + g, solves);
       switch (a.mode) {
         case GAP_ACC: k_decide_epilogue<D, GAP_ACC><<<blocks, kDecideThreads, 0, s>>>(e); break;
         case GAP_PLAIN:
@@ -280,7 +283,7 @@ int launch_fused(const FusedArgs& a00, hipStream_t s, int tile_rows, int engine)
         default: k_decide_epilogue<D, ADMM><<<blocks, kDecideThreads, 0, s>>>(e); break;
       }
     } else {
-      k_decide<D><<<unsigned(a.T), kDecideThreads, 0, s>>>(a);
+      k_decide<D><<<dim3(unsigned(a.T), solves), kDecideThreads, 0, s>>>(a);
     }
     SCIGAP_LAUNCH_CHECK("early-exit decision launch");
   }
@@ -560,36 +563,64 @@ size_t scigap_solve_workspace_bytes(const scigap_params* p) {
   return carve(p, nullptr).bytes;
 }
 
-int scigap_solve(const scigap_params* p, const float* y, const float* phi, const float* phi_sum,
-                 const float* x0, float* x_out, const float* truth, double* sq_err, int* stats,
-                 void* workspace, size_t workspace_bytes, void* stream) {
-  clear_error();
+namespace {
+
+// `solves` reconstructions of one shape, packed one after another in every
+// array, each with a workspace of align256(carve(p).bytes).  The fused
+// iterations of all of them share their launches; other paths (no or deep TV,
+// the split-launch engines) run one solve after another.
+int run_solves(const scigap_params* p, int solves, const float* y, const float* phi,
+               const float* phi_sum, const float* x0, float* x_out, const float* truth,
+               double* sq_err, int* stats, void* workspace, size_t workspace_bytes,
+               void* stream, bool first = true) {
   if (int rc = check_params(p)) return rc;
   if (!y || !phi || !phi_sum || !x_out) return fail(SCIGAP_ENULL, "scigap_solve: null input/output");
   if (truth && !sq_err) return fail(SCIGAP_ENULL, "scigap_solve: truth given without sq_err");
+  if (solves < 1) return fail(SCIGAP_EINVAL, "scigap_solve: the number of solves must be >= 1");
   const int64_t N = p->H * p->W, T = p->T;
-  const size_t vol = size_t(N * T) * 4;
-  if (x0 && overlaps(x0, vol, x_out, vol)) return fail(SCIGAP_EALIAS, "x0 overlaps x_out");
-  if (overlaps(x_out, vol, y, N * 4) || overlaps(x_out, vol, phi, vol) ||
-      overlaps(x_out, vol, phi_sum, N * 4))
+  const size_t vol = size_t(N * T) * 4, vols = vol * solves, planes = size_t(N) * 4 * solves;
+  if (x0 && overlaps(x0, vols, x_out, vols)) return fail(SCIGAP_EALIAS, "x0 overlaps x_out");
+  if (overlaps(x_out, vols, y, planes) || overlaps(x_out, vols, phi, vols) ||
+      overlaps(x_out, vols, phi_sum, planes))
     return fail(SCIGAP_EALIAS, "x_out overlaps an input");
   Workspace ws = carve(p, static_cast<char*>(workspace));
-  if (!workspace || workspace_bytes < ws.bytes)
-    return fail(SCIGAP_EWORKSPACE, "workspace needs %zu bytes, got %zu", ws.bytes, workspace_bytes);
-  if (overlaps(workspace, ws.bytes, x_out, vol)) return fail(SCIGAP_EALIAS, "workspace overlaps x_out");
-  // The tile loads read float2 pairs; keep every plane 8-byte aligned.
-  if ((reinterpret_cast<uintptr_t>(x_out) | reinterpret_cast<uintptr_t>(phi) |
-       reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(x0)) % 8 != 0)
+  const size_t ws_each = align256(ws.bytes), need = ws_each * (solves - 1) + ws.bytes;
+  if (!workspace || workspace_bytes < need)
+    return fail(SCIGAP_EWORKSPACE, "workspace needs %zu bytes, got %zu", need, workspace_bytes);
+  if (overlaps(workspace, need, x_out, vols)) return fail(SCIGAP_EALIAS, "workspace overlaps x_out");
+  // Images of even width are read in float2 pairs; keep their planes 8-byte
+  // aligned.  (The later solves of a group start at an odd element only when
+  // H*W is odd, as the odd frames of any such volume do.)
+  if (first && (reinterpret_cast<uintptr_t>(x_out) | reinterpret_cast<uintptr_t>(phi) |
+                reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(x0)) % 8 != 0)
     return fail(SCIGAP_EINVAL, "device buffers must be 8-byte aligned");
 
   const int D = p->tv_iter_max - 1;
   const bool deep = D > kMaxFused;
   const int deep_depth = deep ? tuned_tv_depth(p->H, p->W, p->T, p->tv_iter_max) : 0;
   int tile_rows = p->tile_rows, engine = p->engine;
-  if (tile_rows == 0 && engine == 0) tuned_solve_config(*p, &tile_rows, &engine);
+  if (solves == 1 && tile_rows == 0 && engine == 0) tuned_solve_config(*p, &tile_rows, &engine);
   hipStream_t s = as_stream(stream);
   const int K = p->iters;
   const int mode = solver_mode(*p);
+  if (solves > 1) {
+    const bool shared_launches = D > 0 && !deep && K > 0 &&
+                                 (engine == 0 || engine == 1 || engine == 6) && solves <= 65535 &&
+                                 int64_t(max_slot_tiles(D, int(p->H), int(p->W))) * kMaxParts *
+                                         solves < (int64_t(1) << 31) - 8;
+    if (!shared_launches) {
+      for (int b = 0; b < solves; ++b) {
+        const size_t o = size_t(b) * N, v = o * T;
+        if (int rc = run_solves(p, 1, y + o, phi + v, phi_sum + o, x0 ? x0 + v : nullptr,
+                                x_out + v, truth ? truth + v : nullptr,
+                                sq_err ? sq_err + size_t(b) * K : nullptr,
+                                stats ? stats + size_t(b) * K : nullptr,
+                                static_cast<char*>(workspace) + b * ws_each, ws.bytes, stream, false))
+          return rc;
+      }
+      return SCIGAP_OK;
+    }
+  }
   if (K == 0) {
     // No iterations: x = x0 or At(y).
     if (x0) {
@@ -598,21 +629,25 @@ int scigap_solve(const scigap_params* p, const float* y, const float* phi, const
     }
     return scigap_adjoint(y, phi, x_out, p->H, p->W, T, stream);
   }
+  const size_t ws_floats = ws_each / 4;
   if (!deep && D > 0) {
     // early-stop counters of every iteration
-    k_fill_i32<<<unsigned((K + 255) / 256), 256, 0, s>>>(ws.st.nexit, K, 0);
+    for (int b = 0; b < solves; ++b)
+      k_fill_i32<<<unsigned((K + 255) / 256), 256, 0, s>>>(ws.st.nexit + ws_floats * b, K, 0);
     SCIGAP_LAUNCH_CHECK("counter fill");
   }
   if (truth)
-    if (int rc = fill_f64(sq_err, K, 0.0, s)) return rc;
+    if (int rc = fill_f64(sq_err, K * solves, 0.0, s)) return rc;
   if (stats) {
-    k_fill_i32<<<(K + 255) / 256, 256, 0, s>>>(stats, K, 0);
+    k_fill_i32<<<unsigned((int64_t(K) * solves + 255) / 256), 256, 0, s>>>(stats, K * solves, 0);
     SCIGAP_LAUNCH_CHECK("stats fill");
   }
-  {
+  for (int b = 0; b < solves; ++b) {
+    const size_t o = size_t(b) * N, v = o * T, w = ws_floats * b;
     ProfScope ps("init", s);
-    k_init<<<grid_pixels(N), 256, 0, s>>>(x0, phi, y, phi_sum, ws.st.r[0], ws.st.y1[0], N, int(T),
-                                          mode, float(p->gamma));
+    k_init<<<grid_pixels(N), 256, 0, s>>>(x0 ? x0 + v : nullptr, phi + v, y + o, phi_sum + o,
+                                          ws.st.r[0] + w, ws.st.y1[0] + w, N, int(T), mode,
+                                          float(p->gamma));
   }
   SCIGAP_LAUNCH_CHECK("init launch");
 
@@ -620,6 +655,13 @@ int scigap_solve(const scigap_params* p, const float* y, const float* phi, const
   for (int k = 0; k < fused_iters; ++k) {
     FusedArgs a = iteration_args(*p, k, p->H, p->W, T, y, phi, phi_sum, x0, x_out, truth, sq_err,
                                  stats, ws.st);
+    if (solves > 1) {
+      a.solves = solves;
+      a.iters = K;
+      a.ws = ws_floats;
+      a.x_in_b = a.x_in == ws.st.xbuf ? ws_floats : size_t(N) * T;
+      a.x_out_b = a.x_out == ws.st.xbuf ? ws_floats : size_t(N) * T;
+    }
     if (D == 0) {
       k_project<<<grid_pixels(N), 256, 0, s>>>(a);
       SCIGAP_LAUNCH_CHECK("projection launch");
@@ -653,14 +695,42 @@ int scigap_solve(const scigap_params* p, const float* y, const float* phi, const
   if (mode == ADMM) {
     // x_{K-1} = theta_{K-1} + b_{K-1} + lambda*r_{K-1}*Phi.
     const bool fy = (K == 1 && !x0);
-    const float* th = K == 1 ? x0 : state_buffer(*p, ws.st, x_out, K - 1);
-    k_admm_final<<<grid_pixels(N), 256, 0, s>>>(th, K == 1 ? nullptr : ws.st.bbuf,
-                                                ws.st.r[(K - 1) & 1], phi, y, x_out, truth,
-                                                truth ? sq_err + (K - 1) : nullptr, N, int(T),
-                                                p->lambda_, fy ? 1 : 0);
+    for (int b = 0; b < solves; ++b) {
+      const size_t o = size_t(b) * N, v = o * T, w = ws_floats * b;
+      const float* th = K == 1 ? x0 : state_buffer(*p, ws.st, x_out, K - 1);
+      if (th) th += th == ws.st.xbuf ? w : v;
+      k_admm_final<<<grid_pixels(N), 256, 0, s>>>(
+          th, K == 1 ? nullptr : ws.st.bbuf + w, ws.st.r[(K - 1) & 1] + w, phi + v, y + o,
+          x_out + v, truth ? truth + v : nullptr,
+          truth ? sq_err + size_t(b) * K + (K - 1) : nullptr, N, int(T), p->lambda_, fy ? 1 : 0);
+    }
     SCIGAP_LAUNCH_CHECK("admm final launch");
   }
   return SCIGAP_OK;
+}
+
+}  // namespace
+
+int scigap_solve(const scigap_params* p, const float* y, const float* phi, const float* phi_sum,
+                 const float* x0, float* x_out, const float* truth, double* sq_err, int* stats,
+                 void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  return run_solves(p, 1, y, phi, phi_sum, x0, x_out, truth, sq_err, stats, workspace,
+                    workspace_bytes, stream);
+}
+
+size_t scigap_solve_many_workspace_bytes(const scigap_params* p, int solves) {
+  if (!p || solves < 1 || check_params(p) != SCIGAP_OK) return 0;
+  return align256(carve(p, nullptr).bytes) * size_t(solves);
+}
+
+int scigap_solve_many(const scigap_params* p, int solves, const float* y, const float* phi,
+                      const float* phi_sum, const float* x0, float* x_out, const float* truth,
+                      double* sq_err, int* stats, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+  clear_error();
+  return run_solves(p, solves, y, phi, phi_sum, x0, x_out, truth, sq_err, stats, workspace,
+                    workspace_bytes, stream);
 }
 
 size_t scigap_tv_workspace_bytes_depth(int64_t H, int64_t W, int64_t T, int n_iter_max,

@@ -121,6 +121,9 @@ SYMBOLS = {
     "scigap_solve_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Params)]),
     "scigap_solve": (_INT, [ctypes.POINTER(Params), _P, _P, _P, _P, _P, _P, _P, _P, _P,
                             ctypes.c_size_t, _P]),
+    "scigap_solve_many_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Params), _INT]),
+    "scigap_solve_many": (_INT, [ctypes.POINTER(Params), _INT, _P, _P, _P, _P, _P, _P, _P, _P, _P,
+                                 ctypes.c_size_t, _P]),
     "scigap_batch_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Params),
                                                        ctypes.POINTER(BatchItem), _INT,
                                                        ctypes.POINTER(BatchOptions)]),

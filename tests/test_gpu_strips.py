@@ -46,3 +46,44 @@ def test_strip_bodies_match_whole_tiles(gpu, H, W, method, accelerate, truth):
     assert torch.equal(stats, statsw)
     # (fp64 sums of the same fp32 terms, added by atomics in any order)
     assert torch.allclose(err, errw, rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("H,W,T", [(1, 1, 1), (5, 7, 3), (24, 130, 2), (70, 317, 5)])
+@pytest.mark.parametrize("method,engine,iters,n", [("gap", 0, 7, 5), ("admm", 6, 7, 5),
+                                                   ("gap", 1, 4, 3), ("admm", 0, 1, 5),
+                                                   ("gap", 3, 3, 5), ("gap", 0, 3, 9),
+                                                   ("gap", 0, 2, 1), ("gap", 0, 0, 5)])
+def test_solves_that_share_launches_match_single_ones(gpu, H, W, T, method, engine, iters, n):
+    """Three solves together against one at a time, with a loose exit tolerance
+    (frames stop early) and with a truth.  The frame split may differ, so yb may
+    round differently: 1e-5, a few hundred fp32 roundings over the iterations."""
+    import torch
+    from pnp_sci import _lib
+    from pnp_sci.synthetic import make_problem
+    prs = [make_problem(H, W, T, seed=H + W + i, p=0.5) for i in range(3)]
+    cat = lambda f: torch.stack([torch.as_tensor(f(q), device="cuda") for q in prs])  # noqa: E731
+    y, phi, ps, tr = (cat(f).contiguous() for f in (lambda q: q.y, lambda q: q.mask_thw,
+                                                    lambda q: q.phi_sum, lambda q: q.truth_thw))
+    p = _lib.Params()
+    gpu.scigap_default_params(p, H, W, T)
+    p.method = _lib.METHOD_ADMM if method == "admm" else _lib.METHOD_GAP
+    p.iters, p.tv_iter_max, p.tv_eps, p.engine = iters, n, 2e-2, engine
+    x = torch.empty_like(phi)
+    err = torch.zeros((3, max(iters, 1)), dtype=torch.float64, device="cuda")
+    stats = torch.zeros((3, max(iters, 1)), dtype=torch.int32, device="cuda")
+    nb = gpu.scigap_solve_many_workspace_bytes(p, 3)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    _lib.check(gpu.scigap_solve_many(p, 3, y.data_ptr(), phi.data_ptr(), ps.data_ptr(), None,
+                                     x.data_ptr(), tr.data_ptr(), err.data_ptr(),
+                                     stats.data_ptr(), ws.data_ptr(), nb, _lib.stream_ptr()))
+    for i in range(3):
+        # (single solves want 8-byte aligned arrays: copies of the slices)
+        yi, fi, si, ti = (v[i].clone() for v in (y, phi, ps, tr))
+        xi, ei = torch.empty_like(fi), torch.zeros_like(err[i])
+        sti = torch.zeros_like(stats[i])
+        _lib.check(gpu.scigap_solve(p, yi.data_ptr(), fi.data_ptr(), si.data_ptr(), None,
+                                    xi.data_ptr(), ti.data_ptr(), ei.data_ptr(), sti.data_ptr(),
+                                    ws.data_ptr(), nb, _lib.stream_ptr()))
+        assert torch.equal(stats[i], sti)
+        assert float((x[i] - xi).abs().max()) <= 1e-5
+        assert torch.allclose(err[i], ei, rtol=1e-4, atol=1e-9)
