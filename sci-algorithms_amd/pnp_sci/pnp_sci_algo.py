@@ -195,15 +195,27 @@ def _run(method, y, Phi_sum, A, At, *, _lambda, accelerate, gamma, clip, denoise
         tv_iter_max = 1  # identity denoiser
     sigma, iter_max = _stages(sigma, iter_max)
     iters = int(sum(iter_max))
+    torch = _torch()
+    group = y if isinstance(y, _Blocks) else None
     phi = recover_mask(A, At, y)
     T, H, W = phi.shape
-    yd = to_device(y, "y")
+    yd = hwt_to_thw(to_device(y.array, "y")) if group else to_device(y, "y")
     psd = to_device(Phi_sum, "Phi_sum")
-    if tuple(yd.shape) != (H, W) or tuple(psd.shape) != (H, W):
+    if tuple(yd.shape[-2:]) != (H, W) or tuple(psd.shape) != (H, W) or yd.dim() != 2 + bool(group):
         raise ValueError("y and Phi_sum must be (H,W) = (%d,%d)" % (H, W))
-    x0d = to_device_thw(x0, "x0") if x0 is not None else None
+
+    def volume(v, name):  # (T,H,W), or the group's [block][T][H][W]
+        if not group:
+            return to_device_thw(v, name)
+        return to_device_thw(v.array, name).reshape(group.n, T, H, W)
+
+    x0d = volume(x0, "x0") if x0 is not None else None
     want_iqa = show_iqa and X_orig is not None
-    truth = to_device_thw(X_orig, "X_orig") if X_orig is not None else None
+    truth = volume(X_orig, "X_orig") if X_orig is not None else None
+    n = group.n if group else 1
+    if group:
+        phi = phi.expand(n, T, H, W).contiguous()
+        psd = psd.expand(n, H, W).contiguous()
     x, sq, _ = solve_device(yd, phi, psd, method=method, iters=iters, _lambda=_lambda,
                             accelerate=accelerate, gamma=gamma, clip=clip, tv_weight=tv_weight,
                             tv_iter_max=tv_iter_max, tv_eps=tv_eps, x0=x0d,
@@ -211,13 +223,30 @@ def _run(method, y, Phi_sum, A, At, *, _lambda, accelerate, gamma, clip, denoise
                             tv_weight_decay=tv_weight_decay, gamma_decay=gamma_decay)
     psnr_all = []
     if want_iqa:
-        psnr_all = _psnr_from_sq(sq.cpu().tolist(), T * H * W)
-        _print_progress(method.upper(), psnr_all, sigma, iter_max)
+        sq = sq.cpu().tolist()
+        psnr_all = [_psnr_from_sq(e, T * H * W) for e in (sq if group else [sq])]
+        _print_progress(method.upper(), psnr_all[0], sigma, iter_max)
     psnr_, ssim_ = [], []
+    x, truth = (None if v is None else v.reshape(n * T, H, W) for v in (x, truth))
     if X_orig is not None:
         psnr_ = psnr_frames(truth, x)
         ssim_ = ssim_frames(truth, x)  # raises for frames under 7x7, as the reference does
-    return to_host_like(thw_to_hwt(x), y), psnr_, ssim_, psnr_all
+    for i in range(1, n):
+        group.on_block(i)
+        if want_iqa:
+            _print_progress(method.upper(), psnr_all[i], sigma, iter_max)
+    out = to_host_like(thw_to_hwt(x), y.array if group else y)
+    return out, psnr_, ssim_, (psnr_all if group else psnr_all[0] if psnr_all else [])
+
+
+class _Blocks:
+    """The arrays of `n` coded-frame blocks of one shape and mask, side by side in
+    the last dimension, which `_run` solves together (as `y`, `x0` and
+    `X_orig`).  Its results are side by side too, psnr_all a list per block;
+    ``on_block(i)`` runs before the progress lines of block i > 0."""
+
+    def __init__(self, array, n, on_block=None):
+        self.array, self.n, self.on_block = array, n, on_block
 
 
 def gap_denoise(y, Phi_sum, A, At, _lambda=1, accelerate=True,
@@ -352,40 +381,63 @@ def admmdenoise_cacti(meas, mask, A, At, projmeth='admm', v0=None, orig=None,
     begin = time.time()
     t_ = 0.0
     msum_host = msum.cpu().numpy()
-    for kf in range(nframe):
+
+    def announce(kf):
         print('%s-%s Reconstruction coded frame block %2d of %2d ...'
               % (projmeth.upper(), args['denoiser'].upper(), kf + 1, nframe))
+
+    def flipped(kf):
+        return ((maskdirection.lower() == 'updown' and (kf + iframe) % 2 == 1) or
+                (maskdirection.lower() == 'downup' and (kf + iframe) % 2 == 0))
+
+    # Blocks are independent solves of one shape: groups of them share their
+    # launches (one block of 256x256x8 fills a tenth of the GPU).
+    voxels = H * W * T
+    per_group = 1
+    if voxels <= _SHARED_SOLVE_VOXELS:
+        per_group = max(1, min(2 * _SHARED_SOLVE_VOXELS // voxels, 4096 // T))
+    for k0 in range(0, nframe, per_group):
+        ks = range(k0, min(k0 + per_group, nframe))
+        announce(k0)
+        n, lo, hi = len(ks), iframe + k0, iframe + ks[-1] + 1
+        pack = lambda v: v if n == 1 else _Blocks(  # noqa: E731
+            v, n, lambda i: announce(k0 + i))
         orig_k = None
         if orig is not None:
-            orig_k = np.asarray(orig[..., (kf + iframe) * nmask:(kf + iframe + 1) * nmask]) / MAXB
-        meas_k = np.asarray(meas[..., kf + iframe]) / MAXB
-        flip = ((maskdirection.lower() == 'updown' and (kf + iframe) % 2 == 1) or
-                (maskdirection.lower() == 'downup' and (kf + iframe) % 2 == 0))
+            orig_k = pack(np.asarray(orig[..., lo * nmask:hi * nmask]) / MAXB)
+        y_k = np.asarray(meas[..., lo] if n == 1 else meas[..., lo:hi]) / MAXB
         v0_k = None
         if v0 is not None:
-            v0_k = np.asarray(v0[:, :, kf * nmask:(kf + 1) * nmask])
-            if flip:
-                v0_k = v0_k[..., ::-1]
+            v0_k = np.asarray(v0[:, :, k0 * nmask:(ks[-1] + 1) * nmask])
+            if any(flipped(kf) for kf in ks):
+                v0_k = np.concatenate(
+                    [v0_k[..., i * nmask:(i + 1) * nmask][..., ::-1 if flipped(kf) else 1]
+                     for i, kf in enumerate(ks)], axis=-1)
+            v0_k = pack(v0_k)
         if projmeth.lower() == 'admm':
-            res = admm_denoise(meas_k, msum_host, A_b, At_b, x0=v0_k, X_orig=orig_k, **args)
+            res = admm_denoise(pack(y_k), msum_host, A_b, At_b, x0=v0_k, X_orig=orig_k, **args)
         elif projmeth.lower() == 'gap':
-            res = gap_denoise(meas_k, msum_host, A_b, At_b, x0=v0_k, X_orig=orig_k, **args)
+            res = gap_denoise(pack(y_k), msum_host, A_b, At_b, x0=v0_k, X_orig=orig_k, **args)
         else:
             # The reference prints this and then reads the unbound result of
             # the solve (pnp_sci_algo.py:518-529): UnboundLocalError.
             print('Unsupported projection method %s' % projmeth.upper())
             raise UnboundLocalError("local variable 'x_k' referenced before assignment")
         x_k, psnr_k, ssim_k, psnrall_k = res
-        if flip:
-            x_k = x_k[..., ::-1]
-            psnr_k = psnr_k[::-1]
-            ssim_k = ssim_k[::-1]
-            psnrall_k = psnrall_k[::-1]
+        if n == nframe and x_k.dtype == x_.dtype:
+            x_ = x_k  # the whole result as it came from the device
+        else:
+            x_[..., k0 * nmask:(k0 + n) * nmask] = x_k
+        for i, kf in enumerate(ks):
+            part = slice(i * nmask, (i + 1) * nmask)
+            step = -1 if flipped(kf) else 1
+            if step < 0:
+                cols = slice(kf * nmask, (kf + 1) * nmask)
+                x_[..., cols] = x_[..., cols][..., ::-1].copy()
+            psnr_.extend(psnr_k[part][::step])
+            ssim_.extend(ssim_k[part][::step])
+            psnrall_.append((psnrall_k if n == 1 else psnrall_k[i] if psnrall_k else [])[::step])
         t_ = time.time() - begin
-        x_[..., kf * nmask:(kf + 1) * nmask] = x_k
-        psnr_.extend(psnr_k)
-        ssim_.extend(ssim_k)
-        psnrall_.append(psnrall_k)
     return x_, t_, psnr_, ssim_, psnrall_
 
 

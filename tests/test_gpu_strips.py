@@ -87,3 +87,37 @@ def test_solves_that_share_launches_match_single_ones(gpu, H, W, T, method, engi
         assert torch.equal(stats[i], sti)
         assert float((x[i] - xi).abs().max()) <= 1e-5
         assert torch.allclose(err[i], ei, rtol=1e-4, atol=1e-9)
+
+
+@pytest.mark.parametrize("projmeth,direction", [("gap", "plain"), ("admm", "updown"),
+                                                ("gap", "downup")])
+@pytest.mark.parametrize("H,W,T,F", [(24, 130, 3, 1), (7, 9, 2, 5), (33, 40, 4, 3)])
+def test_coded_frame_blocks_together_match_one_at_a_time(gpu, capsys, monkeypatch, projmeth,
+                                                         direction, H, W, T, F):
+    """The driver with groups of blocks against the same driver one block at a
+    time: results, progress lines and their order."""
+    import numpy as np
+    import pnp_sci
+    from pnp_sci import pnp_sci_algo
+    from pnp_sci.synthetic import truth_video
+    rng = np.random.default_rng(H + F)
+    mask = (rng.random((H, W, T)) < 0.5).astype(np.float32)
+    orig = (truth_video(rng, H, W, T * F) * 255).astype(np.float32)
+    meas = np.stack([(orig[..., f * T:(f + 1) * T] * mask).sum(2) for f in range(F)], -1)
+    v0 = rng.random((H, W, T * F)).astype(np.float32)
+    for warm in (None, v0):
+        runs = []
+        for voxels in (1 << 25, 0):
+            monkeypatch.setattr(pnp_sci_algo, "_SHARED_SOLVE_VOXELS", voxels)
+            runs.append((pnp_sci.admmdenoise_cacti(
+                meas, mask, lambda v: pnp_sci.A_(v, mask), lambda v: pnp_sci.At_(v, mask),
+                projmeth=projmeth, v0=warm, orig=orig, nframe=F, MAXB=255.,
+                maskdirection=direction, denoiser="tv", iter_max=6), capsys.readouterr().out))
+        (x, _, p, s, pa), text = runs[0]
+        (xw, _, pw, sw, paw), textw = runs[1]
+        assert x.shape == xw.shape and x.dtype == xw.dtype and x.flags.c_contiguous
+        assert np.max(np.abs(x - xw)) <= 1e-5
+        assert np.allclose(p, pw, atol=1e-2) and np.allclose(s, sw, atol=1e-4)
+        assert np.allclose(pa, paw, atol=1e-2)
+        strip = lambda t: [line.split("PSNR")[0] for line in t.splitlines()]  # noqa: E731
+        assert strip(text) == strip(textw)
