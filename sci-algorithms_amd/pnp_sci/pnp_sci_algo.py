@@ -101,6 +101,14 @@ def solve_device(y, phi, phi_sum, *, method="gap", iters=50, _lambda=1.0, accele
     torch = _torch()
     lead = tuple(phi.shape[:-3])
     T, H, W = phi.shape[-3:]
+    if lead:  # the solves' arrays are addressed by their distance: all of it must be there
+        for v, want in ((y, (H, W)), (phi, (T, H, W)), (phi_sum, (H, W)), (x0, (T, H, W)),
+                        (truth, (T, H, W))):
+            if v is not None and (len(lead) > 1 or tuple(v.shape) != lead + want or
+                                  not v.is_contiguous()):
+                raise ValueError("solves that share launches need contiguous tensors with one "
+                                 "leading dimension: got %s, expected %s"
+                                 % (tuple(v.shape), lead + want))
     p = _lib.Params()
     L = _lib.lib()
     L.scigap_default_params(p, H, W, T)
@@ -201,13 +209,17 @@ def _run(method, y, Phi_sum, A, At, *, _lambda, accelerate, gamma, clip, denoise
     T, H, W = phi.shape
     yd = hwt_to_thw(to_device(y.array, "y")) if group else to_device(y, "y")
     psd = to_device(Phi_sum, "Phi_sum")
-    if tuple(yd.shape[-2:]) != (H, W) or tuple(psd.shape) != (H, W) or yd.dim() != 2 + bool(group):
+    lead = (group.n,) if group else ()
+    if tuple(yd.shape) != lead + (H, W) or tuple(psd.shape) != (H, W):
         raise ValueError("y and Phi_sum must be (H,W) = (%d,%d)" % (H, W))
 
     def volume(v, name):  # (T,H,W), or the group's [block][T][H][W]
         if not group:
             return to_device_thw(v, name)
-        return to_device_thw(v.array, name).reshape(group.n, T, H, W)
+        vd = to_device_thw(v.array, name)
+        if tuple(vd.shape) != (group.n * T, H, W):
+            raise ValueError("%s must hold %d frames of %dx%d" % (name, group.n * T, H, W))
+        return vd.reshape(group.n, T, H, W)
 
     x0d = volume(x0, "x0") if x0 is not None else None
     want_iqa = show_iqa and X_orig is not None
@@ -348,6 +360,16 @@ def gap_denoise_bayer(y_bayer, Phi_bayer, _lambda=1, accelerate=True, denoiser='
     return to_host_like(x_bayer, Phi_bayer), psnr_, ssim_, psnr_all
 
 
+def _planes(stack, lo, hi):
+    """Planes lo to hi - 1 of the last axis by the rules of an index: beyond the
+    stack is an IndexError (a slice would end short), negative counts from its
+    end."""
+    planes = [stack[..., i] for i in range(lo, hi)]
+    if lo >= 0:
+        return np.asarray(stack[..., lo:hi])
+    return np.stack([np.asarray(v) for v in planes], axis=-1)
+
+
 def admmdenoise_cacti(meas, mask, A, At, projmeth='admm', v0=None, orig=None,
                       iframe=0, nframe=1, MAXB=1., maskdirection='plain', **args):
     """Per-coded-frame driver (pnp_sci_algo.py:479-534).
@@ -405,7 +427,7 @@ def admmdenoise_cacti(meas, mask, A, At, projmeth='admm', v0=None, orig=None,
         orig_k = None
         if orig is not None:
             orig_k = pack(np.asarray(orig[..., lo * nmask:hi * nmask]) / MAXB)
-        y_k = np.asarray(meas[..., lo] if n == 1 else meas[..., lo:hi]) / MAXB
+        y_k = np.asarray(meas[..., lo] if n == 1 else _planes(meas, lo, hi)) / MAXB
         v0_k = None
         if v0 is not None:
             v0_k = np.asarray(v0[:, :, k0 * nmask:(ks[-1] + 1) * nmask])
