@@ -285,10 +285,12 @@ def admm_denoise(y, Phi_sum, A, At, _lambda=1, gamma=0.01,
                 x0=x0, X_orig=X_orig, show_iqa=show_iqa)
 
 
-# Sub-grids of up to this many voxels (H*W*T) are solved together: four of
-# 512x512x10 take 3.1 ms for 50 iterations instead of 5.5.  A larger one fills
-# the GPU by itself, and one workspace is enough for all four in turn.
-_SHARED_SOLVE_VOXELS = 1 << 25
+# Sub-grids of up to this many voxels (H*W*T) are solved together.  A larger one
+# fills the GPU by itself, and one workspace is enough for all four in turn.
+# (20 iterations, together / in turn: 0.73 / 1.6 ms for sub-grids of 256x256x8,
+# 1.40 / 2.34 of 512x512x10, 7.8 / 8.7 of 2048x1024x8, 10.0 / 9.3 of
+# 1024x1024x20, 14.7 / 12.9 of 2048x2048x8.)
+_SHARED_SOLVE_VOXELS = 1 << 24
 
 
 def gap_denoise_bayer(y_bayer, Phi_bayer, _lambda=1, accelerate=True, denoiser='tv',
@@ -325,27 +327,36 @@ def gap_denoise_bayer(y_bayer, Phi_bayer, _lambda=1, accelerate=True, denoiser='
         v = v.permute((1, 3, 4, 0, 2) if v.dim() == 5 else (1, 3, 0, 2))
         return v.reshape((4,) + tuple(v.shape[2:])).contiguous()
 
-    y_c, phi_c = split(yd), split(phid)
-    ps_c = torch.empty((4, H, W), dtype=torch.float32, device=phid.device)
-    for c in range(4):
-        _lib.check(L.scigap_phi_sum(phi_c[c].data_ptr(), ps_c[c].data_ptr(), H, W, T,
-                                    _lib.stream_ptr()))
-    x0_c = split(x0d) if x0d is not None else None
-    tr_c = split(truth) if want_iqa else None
+    def take(v, c):  # one sub-grid, frame-major, in a tensor of its own
+        v = v[c >> 1::2, c & 1::2].contiguous()
+        return hwt_to_thw(v) if v.dim() == 3 else v
+
+    def frame_sum(phi):
+        ps = torch.empty((H, W), dtype=torch.float32, device=phid.device)
+        _lib.check(L.scigap_phi_sum(phi.data_ptr(), ps.data_ptr(), H, W, T, _lib.stream_ptr()))
+        return ps
+
+    x0d = x0d[..., :nmask] if x0d is not None else None
     opts = dict(method="gap", iters=iters, _lambda=_lambda, accelerate=accelerate,
                 tv_weight=tv_weight, tv_iter_max=tv_iter_max)
     if T * H * W <= _SHARED_SOLVE_VOXELS:
-        x_c, sq, _ = solve_device(y_c, phi_c, ps_c, x0=x0_c, truth=tr_c, **opts)
+        phi_c = split(phid)
+        x_c, sq, _ = solve_device(split(yd), phi_c, torch.stack([frame_sum(f) for f in phi_c]),
+                                  x0=split(x0d) if x0d is not None else None,
+                                  truth=split(truth) if want_iqa else None, **opts)
         sq_total = sq.sum(0) if sq is not None else None
+        x_bayer = x_c.reshape(2, 2, T, H, W).permute(3, 0, 4, 1, 2).reshape(nrow, ncol, nmask)
     else:
-        x_c, sq_total = torch.empty_like(phi_c), None
+        x_bayer = torch.empty((nrow, ncol, nmask), dtype=torch.float32, device=phid.device)
+        sq_total = None
         for c in range(4):
-            x_c[c], sq, _ = solve_device(y_c[c], phi_c[c], ps_c[c],
-                                         x0=x0_c[c] if x0_c is not None else None,
-                                         truth=tr_c[c] if tr_c is not None else None, **opts)
+            phi_c = take(phid, c)
+            x_c, sq, _ = solve_device(take(yd, c), phi_c, frame_sum(phi_c),
+                                      x0=take(x0d, c) if x0d is not None else None,
+                                      truth=take(truth, c) if want_iqa else None, **opts)
+            x_bayer[c >> 1::2, c & 1::2] = thw_to_hwt(x_c)
             if sq is not None:
                 sq_total = sq if sq_total is None else sq_total + sq
-    x_bayer = x_c.reshape(2, 2, T, H, W).permute(3, 0, 4, 1, 2).reshape(nrow, ncol, nmask)
     psnr_all = []
     if want_iqa:
         psnr_all = _psnr_from_sq(sq_total.cpu().tolist(), nrow * ncol * nmask)
@@ -413,11 +424,13 @@ def admmdenoise_cacti(meas, mask, A, At, projmeth='admm', v0=None, orig=None,
                 (maskdirection.lower() == 'downup' and (kf + iframe) % 2 == 0))
 
     # Blocks are independent solves of one shape: groups of them share their
-    # launches (one block of 256x256x8 fills a tenth of the GPU).
+    # launches (one block of 256x256x8 fills a tenth of the GPU) and their
+    # transfers and conversions, which gain at larger sizes too (20 iterations
+    # of two blocks of 2048x1024x8: 21 ms, one at a time 42).
     voxels = H * W * T
     per_group = 1
-    if voxels <= _SHARED_SOLVE_VOXELS:
-        per_group = max(1, min(2 * _SHARED_SOLVE_VOXELS // voxels, 4096 // T))
+    if voxels <= 2 * _SHARED_SOLVE_VOXELS:
+        per_group = max(1, min(4 * _SHARED_SOLVE_VOXELS // voxels, 4096 // T))
     for k0 in range(0, nframe, per_group):
         ks = range(k0, min(k0 + per_group, nframe))
         announce(k0)
