@@ -125,32 +125,31 @@ __global__ void __launch_bounds__(TT * 8) k_transpose(const float* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// Kernels on the reference's (H,W,T) layout.  A block takes P = blockDim.x
-// consecutive pixels, that is P*T consecutive floats: it moves them with
-// 16-byte accesses in memory order and hands them to the pixels (or frames)
-// through LDS, padded by one element every 32 so that reading with a stride
-// of T meets the banks evenly.
+// Kernels on the reference's (H,W,T) layout.  A block takes P consecutive
+// pixels, that is P*T consecutive floats: it moves them with 16-byte accesses
+// in memory order and hands them to the pixels (or frames) through LDS, padded
+// by one element every 32 so that reading with a stride of T meets the banks
+// evenly.
 //
 // All are bound by memory, or by their launch.  A_ plus At_ of 256x256x8 on
 // device tensors take 24 us; converting both operands first (six launches
 // instead of two, three times the traffic) they took 55.  A conversion of
-// 1024x1024x8 takes 12.5 us (5.4 TB/s, the rate of a copy); in 32x32 tiles, of
-// which 8 frames fill a quarter, 32.7.
+// 1024x1024x8 takes 11 us (6 TB/s, with what the caches hold); in 32x32 tiles, of
+// which 8 frames fill a quarter, 35.
 // ---------------------------------------------------------------------------
 
 __host__ __device__ inline int pad32(int e) { return e + (e >> 5); }
 
-// Pixels of a block for `bytes` of LDS per frame of a pixel: the most that
-// leave room for several blocks on a CU; 0 when not even one wave's pixels fit
-// (more than 120 frames of products, 240 of pixels): then each thread reads its
-// own pixel, or the 32x32 tiles of k_transpose run, which such frame counts fill.
-inline int hwt_pixels(int64_t T, int bytes) {
-  for (int P : {256, 128, 64})
-    if (int64_t(P) * T * bytes <= (P == 64 ? 60 : 40) * 1024) return P;
-  return 0;
-}
 inline size_t hwt_lds(int P, int64_t T, int bytes) {
   return size_t(pad32(int(P * T)) + 1) * size_t(bytes);
+}
+
+// Pixels of a block of k_forward_hwt: the most whose products leave room for
+// several blocks on a CU; 0 when not even one wave's fit.
+inline int forward_pixels(int64_t T) {
+  for (int P : {256, 128, 64})
+    if (int64_t(P) * T * 8 <= (P == 64 ? 60 : 40) * 1024) return P;
+  return 0;
 }
 
 // y = sum_t x_t * phi_t on (H,W,T) arrays: exact products in fp64, summed in
@@ -187,17 +186,32 @@ __global__ void __launch_bounds__(256) k_forward_hwt(const float* __restrict__ x
   }
 }
 
-// The same for frame counts whose products do not fit the LDS.
+// The same for frame counts whose products do not fit the LDS: kChunk frames
+// at a time, so that lanes read runs of a pixel's frames and not one frame each
+// (512x512x160: 1130 us that way).
+constexpr int kChunk = 16;
 __global__ void __launch_bounds__(kThreads) k_forward_hwt_many(const float* __restrict__ x,
                                                                const float* __restrict__ phi,
                                                                float* __restrict__ y, int64_t N,
                                                                int T) {
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < N;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    double s = 0.0;
-    for (int t = 0; t < T; ++t) s = acc_prod(x[i * T + t], phi[i * T + t], s);
-    y[i] = float(s);
+  __shared__ double prod[kThreads][kChunk + 1];
+  const int tid = threadIdx.x;
+  const int64_t p0 = int64_t(blockIdx.x) * kThreads;
+  const int np = int(p0 + kThreads <= N ? kThreads : N - p0);
+  double s = 0.0;
+  for (int t0 = 0; t0 < T; t0 += kChunk) {
+    const int nt = T - t0 < kChunk ? T - t0 : kChunk;
+    for (int i = tid; i < np * kChunk; i += kThreads) {
+      const int p = i / kChunk, t = i % kChunk;
+      const int64_t o = (p0 + p) * T + t0 + t;
+      if (t < nt) prod[p][t] = double(x[o]) * double(phi[o]);
+    }
+    __syncthreads();
+    if (tid < np)
+      for (int t = 0; t < nt; ++t) s += prod[tid][t];
+    __syncthreads();
   }
+  if (tid < np) y[p0 + tid] = float(s);
 }
 
 // x_t = y * phi_t on (H,W,T) arrays; 256 pixels a block.
@@ -236,22 +250,33 @@ __global__ void __launch_bounds__(kThreads) k_adjoint_hwt(const float* __restric
   for (int64_t i = done + tid; i < n; i += kThreads) x[base + i] = ys[i / T] * phi[base + i];
 }
 
-// (H,W,T) <-> (T,H,W).  FROM_HWT: src is (H,W,T).  Vector accesses on both
-// sides (host: N % 4 == 0, 16-byte pointers), full blocks only; the last block
-// and other shapes go element by element.
+// (H,W,T) <-> (T,H,W).  FROM_HWT: src is (H,W,T).  P = 1 << logp pixels a
+// block.  Vector accesses on both sides (host: N % 4 == 0, 16-byte pointers),
+// full blocks only; the last block and other shapes go element by element.
 template <bool FROM_HWT, bool VEC>
-__global__ void __launch_bounds__(256) k_relayout(const float* __restrict__ src,
-                                                  float* __restrict__ dst, int64_t N, int T) {
+__global__ void __launch_bounds__(kThreads) k_relayout(const float* __restrict__ src,
+                                                       float* __restrict__ dst, int64_t N, int T,
+                                                       int logp) {
   extern __shared__ float buf[];
-  const int P = blockDim.x, tid = threadIdx.x;
+  const int P = 1 << logp, tid = threadIdx.x;
   const int64_t p0 = int64_t(blockIdx.x) * P, base = p0 * T;
   const int np = int(p0 + P <= N ? P : N - p0), n = np * T;
   const bool vec = VEC && np == P;
-  const int shift = __builtin_ctz(P) - 2;  // P/4 = 1 << shift
+  // The (T,H,W) side: element i is frame i / P of pixel i % P.
+  auto frames = [&](auto&& one) __attribute__((always_inline)) {
+    for (int i = tid; i < P * T; i += kThreads) {
+      const int t = i >> logp, q = i & (P - 1);
+      if (q < np) one(t, q);
+    }
+  };
+  auto frames4 = [&](auto&& four) __attribute__((always_inline)) {
+    for (int i = tid; i < n / 4; i += kThreads)
+      four(i >> (logp - 2), 4 * (i & ((P >> 2) - 1)));
+  };
   if constexpr (FROM_HWT) {
     if (vec) {
       const float4* const v = reinterpret_cast<const float4*>(src + base);
-      for (int i = tid; i < n / 4; i += P) {
+      for (int i = tid; i < n / 4; i += kThreads) {
         const float4 a = v[i];
         buf[pad32(4 * i)] = a.x;
         buf[pad32(4 * i + 1)] = a.y;
@@ -259,40 +284,36 @@ __global__ void __launch_bounds__(256) k_relayout(const float* __restrict__ src,
         buf[pad32(4 * i + 3)] = a.w;
       }
     } else {
-      for (int i = tid; i < n; i += P) buf[pad32(i)] = src[base + i];
+      for (int i = tid; i < n; i += kThreads) buf[pad32(i)] = src[base + i];
     }
     __syncthreads();
-    if (vec) {
-      for (int i = tid; i < n / 4; i += P) {
-        const int t = i >> shift, q = 4 * (i & ((1 << shift) - 1));
-        reinterpret_cast<float4*>(dst + t * N + p0)[q >> 2] =
+    if (vec)
+      frames4([&](int t, int q) {
+        *reinterpret_cast<float4*>(dst + t * N + p0 + q) =
             make_float4(buf[pad32(q * T + t)], buf[pad32((q + 1) * T + t)],
                         buf[pad32((q + 2) * T + t)], buf[pad32((q + 3) * T + t)]);
-      }
-    } else if (tid < np) {
-      for (int t = 0; t < T; ++t) dst[t * N + p0 + tid] = buf[pad32(tid * T + t)];
-    }
+      });
+    else
+      frames([&](int t, int q) { dst[t * N + p0 + q] = buf[pad32(q * T + t)]; });
   } else {
-    if (vec) {
-      for (int i = tid; i < n / 4; i += P) {
-        const int t = i >> shift, q = 4 * (i & ((1 << shift) - 1));
-        const float4 a = reinterpret_cast<const float4*>(src + t * N + p0)[q >> 2];
+    if (vec)
+      frames4([&](int t, int q) {
+        const float4 a = *reinterpret_cast<const float4*>(src + t * N + p0 + q);
         buf[pad32(q * T + t)] = a.x;
         buf[pad32((q + 1) * T + t)] = a.y;
         buf[pad32((q + 2) * T + t)] = a.z;
         buf[pad32((q + 3) * T + t)] = a.w;
-      }
-    } else if (tid < np) {
-      for (int t = 0; t < T; ++t) buf[pad32(tid * T + t)] = src[t * N + p0 + tid];
-    }
+      });
+    else
+      frames([&](int t, int q) { buf[pad32(q * T + t)] = src[t * N + p0 + q]; });
     __syncthreads();
     if (vec) {
       float4* const v = reinterpret_cast<float4*>(dst + base);
-      for (int i = tid; i < n / 4; i += P)
+      for (int i = tid; i < n / 4; i += kThreads)
         v[i] = make_float4(buf[pad32(4 * i)], buf[pad32(4 * i + 1)], buf[pad32(4 * i + 2)],
                            buf[pad32(4 * i + 3)]);
     } else {
-      for (int i = tid; i < n; i += P) dst[base + i] = buf[pad32(i)];
+      for (int i = tid; i < n; i += kThreads) dst[base + i] = buf[pad32(i)];
     }
   }
 }
@@ -480,9 +501,10 @@ int scigap_forward_hwt(const float* x, const float* phi, float* y, int64_t H, in
   if (overlaps(y, N * 4, x, N * T * 4) || overlaps(y, N * 4, phi, N * T * 4))
     return fail(SCIGAP_EALIAS, "scigap_forward_hwt: y overlaps an input");
   hipStream_t s = as_stream(stream);
-  const int P = hwt_pixels(T, 8);
+  const int P = forward_pixels(T);
   if (P == 0) {
-    k_forward_hwt_many<<<grid_for(N), kThreads, 0, s>>>(x, phi, y, N, int(T));
+    k_forward_hwt_many<<<unsigned((N + kThreads - 1) / kThreads), kThreads, 0, s>>>(x, phi, y, N,
+                                                                               int(T));
   } else {
     const unsigned blocks = unsigned((N + P - 1) / P);
     const bool vec =
@@ -515,25 +537,33 @@ int scigap_adjoint_hwt(const float* y, const float* phi, float* x, int64_t H, in
   return SCIGAP_OK;
 }
 
-// (H,W,T) <-> (T,H,W) through k_relayout; false when T does not fit its LDS.
+// (H,W,T) <-> (T,H,W) through k_relayout; false where its pixels do not fit the
+// LDS (over 240 frames) and where the 32x32 tiles of k_transpose, which such
+// frame counts fill, are the better: from about 112 frames on where single
+// elements are moved, since blocks then begin and end inside lines (1001x701x96:
+// 180 us, in tiles 184; x128: 286 / 244; with 16-byte accesses 1024x1024x128:
+// 204 / 276).  Blocks of few pixels, so that 8 or more share a CU: of
+// 1001x701x64 with up to 40 KB of pixels a block 151 us, with as many threads
+// as pixels besides 224, with 10 KB and 256 threads 106.
 static bool relayout(bool from_hwt, const float* src, float* dst, int64_t N, int64_t T,
                      hipStream_t s) {
-  const int P = hwt_pixels(T, 4);
-  if (P == 0) return false;
-  const unsigned blocks = unsigned((N + P - 1) / P);
-  const size_t lds = hwt_lds(P, T, 4);
   const bool vec = N % 4 == 0 &&
                    (reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) % 16 == 0;
+  if (T > (vec ? 240 : 112)) return false;
+  int logp = 8;
+  while (logp > 6 && (T << logp) * 4 > 10 * 1024) --logp;
+  const unsigned blocks = unsigned((N + (1 << logp) - 1) >> logp);
+  const size_t lds = hwt_lds(1 << logp, T, 4);
   if (from_hwt) {
     if (vec)
-      k_relayout<true, true><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+      k_relayout<true, true><<<blocks, kThreads, lds, s>>>(src, dst, N, int(T), logp);
     else
-      k_relayout<true, false><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+      k_relayout<true, false><<<blocks, kThreads, lds, s>>>(src, dst, N, int(T), logp);
   } else {
     if (vec)
-      k_relayout<false, true><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+      k_relayout<false, true><<<blocks, kThreads, lds, s>>>(src, dst, N, int(T), logp);
     else
-      k_relayout<false, false><<<blocks, P, lds, s>>>(src, dst, N, int(T));
+      k_relayout<false, false><<<blocks, kThreads, lds, s>>>(src, dst, N, int(T), logp);
   }
   return true;
 }
