@@ -356,7 +356,8 @@ __global__ void __launch_bounds__(kThreads) k_sq_error(const float* __restrict__
 // Bound by fp64 arithmetic (4.4 cycles an instruction): a lane walks kSR rows
 // of one column with the window's seven row sums of x, y, x^2, y^2 and x*y in
 // registers, so each row costs seven taps, not 49.  253x317x7: 13.4 us,
-// with all 49 taps per centre 33.7.
+// with all 49 taps per centre 33.7.  The walk ends with the last centre:
+// in a stack of small frames most rows of a workgroup are beyond it.
 constexpr int kSW = 4;  // waves per workgroup, one above the other
 constexpr int kSR = 8;  // window centres per lane
 __global__ void __launch_bounds__(64 * kSW) k_ssim(const float* __restrict__ a,
@@ -373,9 +374,9 @@ __global__ void __launch_bounds__(64 * kSW) k_ssim(const float* __restrict__ a,
   const int cc = c < W - 3 ? c : W - 4;             // (lanes beyond add nothing)
   double s = 0.0;
   double ring[7][5];
-  static_for<kSR + 6>([&](auto ic) __attribute__((always_inline)) {
+  auto row_step = [&](auto ic) __attribute__((always_inline)) {
     constexpr int i = decltype(ic)::value;
-    const int row = r0 - 3 + i < H ? r0 - 3 + i : H - 1;
+    const int row = r0 - 3 + i;
     const float* pa = fa + size_t(row) * W + cc - 3;
     const float* pb = fb + size_t(row) * W + cc - 3;
     double q[5] = {};
@@ -406,9 +407,15 @@ __global__ void __launch_bounds__(64 * kSW) k_ssim(const float* __restrict__ a,
       const double a1 = 2 * ux * uy + c1, a2 = 2 * vxy + c2;
       const double b1 = ux * ux + uy * uy + c1, b2 = vx + vy + c2;
       const double v = (a1 * a2) / (b1 * b2);
-      if (r0 - 6 + i < H - 3 && c < W - 3) s += v;
+      if (c < W - 3) s += v;
     }
-  });
+  };
+  if (r0 + kSR <= H - 3)
+    static_for<kSR + 6>(row_step);
+  else  // the last rows, if any
+    static_for<kSR + 6>([&](auto ic) __attribute__((always_inline)) {
+      if (r0 < H - 3 && r0 - 3 + decltype(ic)::value < H) row_step(ic);
+    });
   s = wave_sum(s);
   __shared__ double part[kSW];
   if ((threadIdx.x & 63) == 0) part[w] = s;
