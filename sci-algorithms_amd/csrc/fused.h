@@ -375,6 +375,14 @@ __device__ __forceinline__ void store_owned(float* __restrict__ p, int N, int W,
   }
 }
 
+// This wave's share of the zeroes of the tile's energy slots.
+template <int D, int BY, bool ENERGY>
+__device__ __forceinline__ void zero_energies(float* red) {
+  if constexpr (ENERGY)
+    for (int i = threadIdx.x; i < kEnergyFrames * BY * EnergySlots<D>::kPerWave; i += blockDim.x)
+      red[i] = 0.f;
+}
+
 // One strip (wave) of one tile of one fused outer iteration.  X1 selects the one-barrier TV
 // engine (tv_run_x1).  ENERGY false: no exit test follows and no energies are
 // formed.
@@ -452,6 +460,9 @@ __device__ __forceinline__ void fused_strip(const FusedArgs& a, int tile,
       }
     }
   }
+  // (after the first loads' requests: before them, a workgroup with one frame
+  // held its memory latency that much longer, 2% of the launch at 1500x1500x1)
+  zero_energies<D, BY, ENERGY>(red);
   float err = 0.f;
 
   // Frame t+1's x and Phi are requested before frame t's TV so that their
@@ -677,6 +688,7 @@ __device__ __forceinline__ void fused_strip_empty(const FusedArgs& a, int tile,
   const int lane = threadIdx.x & 63;
   reinterpret_cast<float2*>(sh.eng.xo)[strip * 64 + lane] = make_float2(0.f, 0.f);
   reinterpret_cast<float2*>(sh.eng.xp)[(strip + 1) * 64 + lane] = make_float2(0.f, 0.f);
+  zero_energies<D, BY, ENERGY>(sh.red);
   const int nparts = a.fsplit > 1 ? a.fsplit : 1;
   const int t_lo = (a.T * part) / nparts, T = (a.T * (part + 1)) / nparts - t_lo;
   for (int t = 0; t < T; ++t) {
@@ -712,9 +724,6 @@ __device__ __forceinline__ void fused_tile(const FusedArgs& a, int tile,
                                            FusedLds<D, BY, MR, X1, DMA>& sh, int part = 0) {
   using G = TileGeom<D, BY, MR>;
   if constexpr (!X1) sh.eng.zero_edges();
-  if constexpr (ENERGY)
-    for (int i = threadIdx.x; i < kEnergyFrames * BY * EnergySlots<D>::kPerWave; i += blockDim.x)
-      sh.red[i] = 0.f;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
   const ColPlace cp = col_place(tx, a.tiles_x, a.W, G::LW, G::HC, G::OX);
@@ -815,27 +824,28 @@ __host__ __device__ inline bool tile_inside(int tile, int tiles_x, int H, int W)
 
 // One launch covers interior and border tiles.  PART restricts a launch to
 // one class (1: interior, 2: border; 0: both), so that the interior kernel is
-// allocated registers for its own body only.  With the
+// allocated registers for its own body only.  MANY: several solves share the
+// launch; a kernel of its own, because the arguments of a solve chosen at run
+// time take scalar registers that every strip body is short of (one kernel for
+// both: 66 of them spilled instead of 55 in GAP, 1-2% of the launch for sizes
+// from 253x317x7 to 1024x1024x20).  With the
 // per-iteration error (IQA) the 8-wave kernel is held to 128 VGPRs, the limit
 // for two workgroups per CU (it would take 130-133; with one workgroup per CU
 // a 2048x2048x20 solve takes 48 ms instead of 32).
 template <int D, int BY, int MR, int MODE, bool IQA, bool X1 = false, int PART = 0,
-          bool DMA = false>
+          bool DMA = false, bool MANY = false>
 __global__ void __launch_bounds__(64 * BY)
 __attribute__((amdgpu_waves_per_eu(BY == 8 && D <= 4 && IQA ? 4 : 1))) k_fused(FusedArgs a) {
   __shared__ FusedLds<D, BY, MR, X1, DMA> sh;
   // Work item -> (solve, tile, frame part); the parts of a tile are adjacent,
   // so they run on the same XCD.
   int item = tile_of_block(blockIdx.x, a.per_xcd);
-  if constexpr (PART == 0 && !X1 && MODE != TV_ONLY) {
+  if (item >= a.ntiles) {
+    if constexpr (!MANY) return;
     const int b = item / a.ntiles;
-    if (item >= a.ntiles) {
-      if (b >= a.solves) return;
-      item -= b * a.ntiles;
-      select_solve(a, b);
-    }
-  } else {
-    if (item >= a.ntiles) return;
+    if (b >= a.solves) return;
+    item -= b * a.ntiles;
+    select_solve(a, b);
   }
   const int nparts = a.fsplit > 1 ? a.fsplit : 1;
   const int tile = item / nparts, part = item - tile * nparts;
@@ -900,9 +910,9 @@ __device__ __forceinline__ void decide_frame(const FusedArgs& a, int t) {
 // one round, 7.2 us per launch against 8.8 us for 512 and 11.8 us for 256.
 constexpr int kDecideThreads = 1024;
 
-template <int D>
+template <int D, bool MANY>
 __global__ void __launch_bounds__(kDecideThreads) k_decide(FusedArgs a) {
-  if (blockIdx.y > 0) select_solve(a, blockIdx.y);
+  if (MANY && blockIdx.y > 0) select_solve(a, blockIdx.y);
   decide_frame<D, kDecideThreads>(a, blockIdx.x);
 }
 
@@ -911,9 +921,9 @@ __global__ void __launch_bounds__(kDecideThreads) k_decide(FusedArgs a) {
 // each, the rest run the epilogue over the pixels (the two read different
 // results of the main pass, and the repair after them needs both).  One
 // launch less per outer iteration where launches dominate (small problems).
-template <int D, int MODE>
+template <int D, int MODE, bool MANY>
 __global__ void __launch_bounds__(kDecideThreads) k_decide_epilogue(FusedArgs a) {
-  if (blockIdx.y > 0) select_solve(a, blockIdx.y);
+  if (MANY && blockIdx.y > 0) select_solve(a, blockIdx.y);
   if (blockIdx.x < unsigned(a.T)) {  // workgroup-uniform
     decide_frame<D, kDecideThreads>(a, blockIdx.x);
     return;
@@ -1096,13 +1106,12 @@ constexpr int kStopLds = 1024;
 // For D <= 4 at least 4 waves per SIMD: two 8-wave workgroups per CU
 // (128 VGPRs); deeper tiles need more registers than that.  Runs after
 // k_decide; returns at once when no frame stopped early (the common case).
-template <int D, int BY, int MR, int MODE>
+template <int D, int BY, int MR, int MODE, bool MANY>
 __global__ void __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(D <= 4 ? 4 : 1)))
 k_fused_fix(FusedArgs a) {
   __shared__ FixLds<D, BY, MR> sh;
   __shared__ int s_stop[kStopLds];
-  if constexpr (MODE != TV_ONLY)
-    if (blockIdx.y > 0) select_solve(a, blockIdx.y);
+  if (MANY && blockIdx.y > 0) select_solve(a, blockIdx.y);
   if (*a.nexit == 0) return;  // one scalar load per workgroup
   const int tile = tile_of_block(blockIdx.x, a.per_xcd);
   if (tile >= a.ntiles) return;

@@ -84,6 +84,11 @@ unsigned set_tiles(FusedArgs& a) {
 
 template <int D, int BY, int MODE, bool IQA, bool X1, int PART, bool DMA = false, int MR = 1>
 void launch_kernel(const FusedArgs& a, unsigned grid, hipStream_t s) {
+  if constexpr (PART == 0 && !X1 && !DMA && MODE != TV_ONLY)
+    if (a.solves > 1) {
+      k_fused<D, BY, MR, MODE, IQA, X1, PART, DMA, true><<<grid, 64 * BY, 0, s>>>(a);
+      return;
+    }
   k_fused<D, BY, MR, MODE, IQA, X1, PART, DMA><<<grid, 64 * BY, 0, s>>>(a);
 }
 
@@ -232,6 +237,46 @@ int main_tiles_for(int H, int W, int tile_rows, int engine) {
   }
 }
 
+// The launches after the main pass: the early-exit decision (with the parts'
+// epilogue when the main pass was split into `parts`) and the repair.
+template <int D, int MODE, bool MANY>
+int launch_decide_and_repair(const FusedArgs& a0, int parts, hipStream_t s) {
+  constexpr int FBY = FixShape<D>::BY, MR = FusedShape<D>::MR;
+  FusedArgs a = a0;
+  const unsigned solves = MANY ? unsigned(a.solves) : 1;
+  const dim3 grid(set_tiles<D, FBY, MR>(a), solves);
+  {
+    ProfScope ps("fused_decide", s);
+    bool folded = false;
+    if constexpr (MODE != TV_ONLY)
+      if (parts > 1) {
+        FusedArgs e = a0;
+        e.fsplit = parts;
+        const int64_t N = int64_t(a.H) * a.W;
+        const unsigned g =
+            unsigned(std::min<int64_t>((N + kDecideThreads - 1) / kDecideThreads, 1024));
+        k_decide_epilogue<D, MODE, MANY>
+            <<<dim3(unsigned(a.T) + g, solves), kDecideThreads, 0, s>>>(e);
+        folded = true;
+      }
+    if (!folded) k_decide<D, MANY><<<dim3(unsigned(a.T), solves), kDecideThreads, 0, s>>>(a);
+    SCIGAP_LAUNCH_CHECK("early-exit decision launch");
+  }
+  {
+    ProfScope ps("fused_fix", s);
+    k_fused_fix<D, FBY, MR, MODE, MANY><<<grid, 64 * FBY, 0, s>>>(a);
+  }
+  SCIGAP_LAUNCH_CHECK("fused early-exit launch");
+  return SCIGAP_OK;
+}
+
+template <int D, int MODE>
+int launch_decide_and_repair(const FusedArgs& a, int parts, hipStream_t s) {
+  if constexpr (MODE != TV_ONLY)
+    if (a.solves > 1) return launch_decide_and_repair<D, MODE, true>(a, parts, s);
+  return launch_decide_and_repair<D, MODE, false>(a, parts, s);
+}
+
 template <int D>
 int launch_fused(const FusedArgs& a00, hipStream_t s, int tile_rows, int engine) {
   constexpr int BY = FusedShape<D>::BY, MR = FusedShape<D>::MR;
@@ -262,42 +307,12 @@ int launch_fused(const FusedArgs& a00, hipStream_t s, int tile_rows, int engine)
   // frame can stop early and there is nothing to decide or repair.
   if (!a0.stop) return SCIGAP_OK;
   if (!a0.eslot) return fail(SCIGAP_EINVAL, "early exit without energy slots");
-  FusedArgs a = a0;
-  constexpr int FBY = FixShape<D>::BY;
-  const unsigned solves = unsigned(std::max(a.solves, 1));
-  const dim3 grid(set_tiles<D, FBY, MR>(a), solves);
-  {
-    ProfScope ps("fused_decide", s);
-    if (parts > 1) {
-      FusedArgs e = a0;
-      e.fsplit = parts;
-      const int64_t N = int64_t(a.H) * a.W;
-      const unsigned g =
-          unsigned(std::min<int64_t>((N + kDecideThreads - 1) / kDecideThreads, 1024));
-      const dim3 blocks(unsigned(a.T) + g, solves);
-      switch (a.mode) {
-        case GAP_ACC: k_decide_epilogue<D, GAP_ACC><<<blocks, kDecideThreads, 0, s>>>(e); break;
-        case GAP_PLAIN:
-          k_decide_epilogue<D, GAP_PLAIN><<<blocks, kDecideThreads, 0, s>>>(e);
-          break;
-        default: k_decide_epilogue<D, ADMM><<<blocks, kDecideThreads, 0, s>>>(e); break;
-      }
-    } else {
-      k_decide<D><<<dim3(unsigned(a.T), solves), kDecideThreads, 0, s>>>(a);
-    }
-    SCIGAP_LAUNCH_CHECK("early-exit decision launch");
+  switch (a0.mode) {
+    case GAP_ACC: return launch_decide_and_repair<D, GAP_ACC>(a0, parts, s);
+    case GAP_PLAIN: return launch_decide_and_repair<D, GAP_PLAIN>(a0, parts, s);
+    case ADMM: return launch_decide_and_repair<D, ADMM>(a0, parts, s);
+    default: return launch_decide_and_repair<D, TV_ONLY>(a0, parts, s);
   }
-  {
-    ProfScope ps("fused_fix", s);
-    switch (a.mode) {
-      case GAP_ACC: k_fused_fix<D, FBY, MR, GAP_ACC><<<grid, 64 * FBY, 0, s>>>(a); break;
-      case GAP_PLAIN: k_fused_fix<D, FBY, MR, GAP_PLAIN><<<grid, 64 * FBY, 0, s>>>(a); break;
-      case ADMM: k_fused_fix<D, FBY, MR, ADMM><<<grid, 64 * FBY, 0, s>>>(a); break;
-      default: k_fused_fix<D, FBY, MR, TV_ONLY><<<grid, 64 * FBY, 0, s>>>(a); break;
-    }
-  }
-  SCIGAP_LAUNCH_CHECK("fused early-exit launch");
-  return SCIGAP_OK;
 }
 
 int launch_fused_depth(int D, const FusedArgs& a, hipStream_t s, int tile_rows = 0,
