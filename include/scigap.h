@@ -130,8 +130,9 @@ int scigap_tv_chambolle(const float* image, float* out,
  * at most 6, else row sweeps in passes of 3 to 6 updates (or the depth the
  * autotuner found faster for this shape).  Results do not depend on the
  * depth.  The workspace for a given depth is
- * scigap_tv_workspace_bytes_depth(); depth 0 needs the most for more than 6
- * updates, and runs in chunks of 6 in a workspace sized for another depth. */
+ * scigap_tv_workspace_bytes_depth(); with more than 6 updates one size does for
+ * every depth (explicit depths need a little less; depth 0 runs in chunks in
+ * such a workspace). */
 size_t scigap_tv_workspace_bytes_depth(int64_t H, int64_t W, int64_t T, int n_iter_max,
                                        int depth);
 int scigap_tv_chambolle_depth(const float* image, float* out,
@@ -347,10 +348,12 @@ int scigap_unrolled_backward(const scigap_unrolled* u, const float* lambdas,
 typedef struct scigap_tune_result {
   int tile_rows;      /* chosen fused-kernel tile height (solve)            */
   int engine;         /* chosen fused-kernel engine (solve)                 */
-  int tv_depth;       /* chosen TV fusion depth (TV)                        */
-  int candidates;     /* configurations timed                               */
-  double best_ms;     /* per outer iteration (solve) or per call (TV)       */
-  double default_ms;  /* the same for the first candidate (the default)     */
+  int tv_depth;       /* fastest TV fusion depth (TV)                       */
+  int candidates;     /* configurations or depths timed                     */
+  double best_ms;     /* per outer iteration (solve) or per call (TV) from
+                       * now on                                             */
+  double default_ms;  /* the same before tuning: of the first candidate, or of
+                       * the row sweeps (TV of more than 6 updates)         */
 } scigap_tune_result;
 
 /* Time the fused kernel's tile heights and engines on this problem (`iters`
@@ -363,9 +366,11 @@ int scigap_autotune_solve(const scigap_params* p, const float* y, const float* p
                           void* workspace, size_t workspace_bytes, void* stream,
                           scigap_tune_result* result);
 
-/* Time every TV fusion depth for this shape (workspace of at least
- * scigap_tv_workspace_bytes_depth(H,W,T,n_iter_max,1) bytes), remember the
- * fastest (used by depth 0 for deep TV and by the solvers' deep-TV path).
+/* Time every TV fusion depth for this shape and, with more than 6 updates, the
+ * row sweeps (workspace of at least
+ * scigap_tv_workspace_bytes_depth(H,W,T,n_iter_max,1) bytes), and remember the
+ * fastest depth.  Depth 0 and the solvers' deep-TV path use it where it beat the
+ * sweeps (best_ms < default_ms).  Nothing changes when the call fails.
  * Synchronises `stream`. */
 int scigap_autotune_tv(const float* image, float* out, int64_t H, int64_t W, int64_t T,
                        float weight, float eps, int n_iter_max, void* workspace,

@@ -47,7 +47,7 @@ int tv_chunked(const float* image, float* out, int64_t H, int64_t W, int64_t T, 
 size_t tv_sweep_workspace(int64_t H, int64_t W, int64_t T);
 int tv_sweep(const float* image, float* out, int64_t H, int64_t W, int64_t T, float weight,
              float eps, int n, int* stop_iter, int* early, void* ws, hipStream_t s);
-int tuned_tv_depth(int64_t H, int64_t W, int64_t T, int n);
+int tuned_tv_depth(int64_t H, int64_t W, int64_t T, int n, bool sweep_fits);
 bool tuned_solve_config(const scigap_params& p, int* tile_rows, int* engine);
 
 namespace {
@@ -612,7 +612,7 @@ int run_solves(const scigap_params* p, int solves, const float* y, const float* 
 
   const int D = p->tv_iter_max - 1;
   const bool deep = D > kMaxFused;
-  const int deep_depth = deep ? tuned_tv_depth(p->H, p->W, p->T, p->tv_iter_max) : 0;
+  const int deep_depth = deep ? tuned_tv_depth(p->H, p->W, p->T, p->tv_iter_max, true) : 0;
   int tile_rows = p->tile_rows, engine = p->engine;
   if (solves == 1 && tile_rows == 0 && engine == 0) tuned_solve_config(*p, &tile_rows, &engine);
   hipStream_t s = as_stream(stream);
@@ -758,8 +758,7 @@ size_t scigap_tv_workspace_bytes_depth(int64_t H, int64_t W, int64_t T, int n_it
   if (depth >= D)
     return align256(size_t(T) * D * size_t(max_slot_tiles(D, int(H), int(W))) * 4) +
            align256(size_t(T) * 4) + 256;
-  return depth == 0 ? deep_tv_workspace(H, W, T, n_iter_max)
-                    : tv_chunked_workspace(H, W, T, n_iter_max, D);
+  return deep_tv_workspace(H, W, T, n_iter_max);
 }
 
 size_t scigap_tv_workspace_bytes(int64_t H, int64_t W, int64_t T, int n_iter_max) {
@@ -782,10 +781,9 @@ int scigap_tv_chambolle_depth(const float* image, float* out, int64_t H, int64_t
   const size_t vol = size_t(H * W * T) * 4;
   if (overlaps(image, vol, out, vol)) return fail(SCIGAP_EALIAS, "image and out overlap");
   size_t need = scigap_tv_workspace_bytes_depth(H, W, T, n_iter_max, depth);
-  // A workspace sized for an explicit depth does for depth 0 as well: the
-  // chunks run in it then.
+  // Chunks need less than the sweeps: in a smaller workspace depth 0 runs them.
   bool sweep_fits = true;
-  if (depth == 0 && n_iter_max - 1 > kMaxFused && workspace_bytes < need) {
+  if (n_iter_max - 1 > kMaxFused && workspace_bytes < need) {
     need = tv_chunked_workspace(H, W, T, n_iter_max, n_iter_max - 1);
     sweep_fits = false;
   }
@@ -805,8 +803,7 @@ int scigap_tv_chambolle_depth(const float* image, float* out, int64_t H, int64_t
     }
     return SCIGAP_OK;
   }
-  if (depth == 0) depth = D <= kMaxFused ? D : tuned_tv_depth(H, W, T, n_iter_max);
-  if (depth == 0 && !sweep_fits) depth = kMaxFused;
+  if (depth == 0) depth = D <= kMaxFused ? D : tuned_tv_depth(H, W, T, n_iter_max, sweep_fits);
   if (depth == 0)
     return tv_sweep(image, out, H, W, T, weight, eps, n_iter_max, stop_iter, nullptr, workspace,
                     s);

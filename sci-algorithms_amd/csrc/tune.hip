@@ -7,8 +7,8 @@
 // variable SCIGAP_TUNE_CACHE names a file, entries are loaded from it on
 // first use and every new entry is appended to it, so later processes start
 // tuned.  scigap_solve uses a cached entry when its tile_rows and engine are
-// both 0; scigap_tv_chambolle uses the cached depth for depth 0 (an entry of
-// depth 0 says that the row sweeps beat every depth).
+// both 0; scigap_tv_chambolle uses the cached depth for depth 0 where that
+// depth was timed against the row sweeps and beat them.
 
 #include <hip/hip_runtime.h>
 
@@ -24,11 +24,15 @@
 namespace scigap {
 
 int max_chunk_depth();
+size_t tv_sweep_workspace(int64_t H, int64_t W, int64_t T);
+int tv_sweep(const float* image, float* out, int64_t H, int64_t W, int64_t T, float weight,
+             float eps, int n, int* stop_iter, int* early, void* ws, hipStream_t s);
 int check_params(const scigap_params* p);
 
 namespace {
 
-// kind 0: solve (a = method*2 + accelerate, b = tv_iter_max); kind 1: TV (b = n).
+// kind 0: solve (a = method*2 + accelerate, b = tv_iter_max); kind 1: TV (b = n,
+// engine 1 when `depth` beat the row sweeps; 0 in files older than the sweeps).
 using Key = std::tuple<int, int64_t, int64_t, int64_t, int, int>;
 struct Entry {
   int tile_rows = 0, engine = 0, depth = 0;
@@ -82,12 +86,6 @@ void store(const Key& k, const Entry& e) {
   }
 }
 
-void forget(const Key& k) {
-  std::lock_guard<std::mutex> lock(g_mu);
-  load_locked();
-  g_cache.erase(k);
-}
-
 bool lookup(const Key& k, Entry* e) {
   std::lock_guard<std::mutex> lock(g_mu);
   load_locked();
@@ -136,13 +134,15 @@ double time_on_stream(F&& fn, hipStream_t s, int reps, int* rc) {
 
 }  // namespace
 
-// Tuned TV fusion depth for a deep TV (n - 1 > 6 updates); 0 (row sweeps,
-// tv_sweep.hip) when untuned or when the sweeps were the fastest.
-int tuned_tv_depth(int64_t H, int64_t W, int64_t T, int n) {
+// How depth 0 runs a deep TV (n - 1 > 6 updates): a tuned depth that beat the
+// row sweeps, else 0, the sweeps (tv_sweep.hip).  In a workspace too small for
+// the sweeps the tuned depth, 6 when untuned.
+int tuned_tv_depth(int64_t H, int64_t W, int64_t T, int n, bool sweep_fits) {
   Entry e;
-  if (lookup(Key(1, H, W, T, 0, n), &e) && e.depth >= 1 && e.depth <= max_chunk_depth())
-    return e.depth;
-  return 0;
+  const bool tuned = lookup(Key(1, H, W, T, 0, n), &e) && e.depth >= 1 &&
+                     e.depth <= max_chunk_depth();
+  if (!sweep_fits) return tuned ? e.depth : max_chunk_depth();
+  return tuned && e.engine == 1 ? e.depth : 0;
 }
 
 // Tuned (tile_rows, engine) of a solve shape, if any.
@@ -223,21 +223,6 @@ int scigap_autotune_tv(const float* image, float* out, int64_t H, int64_t W, int
   double def_ms = -1.0;
   int n = 0;
   const int dmax = max_chunk_depth();
-  // The untuned path (depth 0) is not a candidate, but a depth is remembered
-  // only if it beats it.
-  const Key key(1, H, W, T, 0, n_iter_max);
-  forget(key);
-  double untuned_ms = -1.0;
-  if (D > dmax && workspace_bytes >= scigap_tv_workspace_bytes_depth(H, W, T, n_iter_max, 0)) {
-    int rc = SCIGAP_OK;
-    untuned_ms = time_on_stream(
-        [&]() {
-          return scigap_tv_chambolle_depth(image, out, H, W, T, weight, eps, n_iter_max, 0,
-                                           nullptr, workspace, workspace_bytes, stream);
-        },
-        s, 2, &rc);
-    if (rc != SCIGAP_OK) return rc;
-  }
   for (int d = dmax; d >= 1; --d) {
     if (d > D) continue;
     int rc = SCIGAP_OK;
@@ -255,17 +240,27 @@ int scigap_autotune_tv(const float* image, float* out, int64_t H, int64_t W, int
       best.ms = ms;
     }
   }
-  Entry keep = best;
-  if (untuned_ms >= 0.0 && untuned_ms <= best.ms) {
-    keep.depth = 0;
-    keep.ms = untuned_ms;
+  // The row sweeps, what depth 0 runs untuned (the arguments were checked by the
+  // calls above).
+  double best_ms = best.ms;
+  if (D > dmax && workspace_bytes >= tv_sweep_workspace(H, W, T)) {
+    int rc = SCIGAP_OK;
+    def_ms = time_on_stream(
+        [&]() {
+          return tv_sweep(image, out, H, W, T, weight, eps, n_iter_max, nullptr, nullptr, workspace,
+                          s);
+        },
+        s, 2, &rc);
+    if (rc != SCIGAP_OK) return rc;
+    best.engine = best.ms < def_ms ? 1 : 0;
+    if (!best.engine) best_ms = def_ms;
   }
-  store(key, keep);
+  store(Key(1, H, W, T, 0, n_iter_max), best);
   res->tile_rows = 0;
   res->engine = 0;
   res->tv_depth = best.depth;
   res->candidates = n;
-  res->best_ms = best.ms;
+  res->best_ms = best_ms;
   res->default_ms = def_ms;
   return SCIGAP_OK;
 }

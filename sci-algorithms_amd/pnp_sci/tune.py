@@ -3,7 +3,7 @@
 * ``autotune_solve``: tile height x engine of the fused GAP/ADMM-TV kernel,
   timed on the caller's data by ``scigap_autotune_solve``; later solves of
   the same shape with default options use the choice.
-* ``autotune_tv``: the TV fusion depth (dual updates per launch) of
+* ``autotune_tv``: the TV fusion depth (dual updates per launch) or row sweeps of
   ``scigap_tv_chambolle`` for deep TV (``scigap_autotune_tv``).
 * ``autotune_batch``: tile height, persistent grid and queue order of a
   batched plan, timed on the batch itself.
