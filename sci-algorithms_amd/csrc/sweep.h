@@ -183,7 +183,11 @@ struct Rows {
   f2 out[S + 1][kRing];
   Dual q[S + 1][kRing];
   int lim = S;    // LIMIT only; wave-uniform
-  float acc[S];   // 16 times this lane's part of E_u over the owned rows
+  // 16 times this lane's part of E_u over the owned rows: `acc` adds up kSumRows
+  // rows, `tot` those sums, so that no chain of fp32 additions grows with the
+  // strip's height (64 rows: 256 terms in one, up to 3e-6 of their sum).
+  static constexpr int kSumRows = 4;
+  float acc[S] = {}, tot[S] = {};
 
   // Step of row I (its image row and, with FROM_Q, dual row already stored in
   // img[I % kRing], q[0][I % kRing]); `row` is its global row.  FILL: one of
@@ -241,7 +245,15 @@ struct Rows {
     // them into the branch that uses them and keeps every term live until then.
     if constexpr (ENERGY)
 #pragma unroll
-      for (int u = 0; u < S; ++u) compute_here(acc[u]);
+      for (int u = 0; u < S; ++u) {
+        if constexpr (FILL ? I + 1 == kFill : (M + 1) % kSumRows == 0) {
+          tot[u] += acc[u];
+          acc[u] = 0.f;
+          compute_here(tot[u]);
+        } else {
+          compute_here(acc[u]);
+        }
+      }
   }
 
   template <bool OWN, bool CUT>

@@ -122,8 +122,6 @@ __device__ __forceinline__ void pass_strip(const PassArgs& a, int strip, int t, 
   const __amdgpu_buffer_rsrc_t wo = plane_rsrc(a.out + size_t(t) * N, N);
   E rows;
   rows.lim = lim;
-#pragma unroll
-  for (int u = 0; u < S; ++u) rows.acc[u] = 0.f;
   f2 ni[P], n0[P], n1[P];
   auto request = [&](auto pc, int i) __attribute__((always_inline)) {
     constexpr int p = decltype(pc)::value;
@@ -178,7 +176,7 @@ __device__ __forceinline__ void pass_strip(const PassArgs& a, int strip, int t, 
     for (int g = 0; g < S; g += 4) {
       float s[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) s[u] = g + u < S && sp.owner ? rows.acc[g + u < S ? g + u : 0] : 0.f;
+      for (int u = 0; u < 4; ++u) s[u] = g + u < S && sp.owner ? rows.tot[g + u < S ? g + u : 0] : 0.f;
       const float k = wave_sum4(s);
       const int e = g + 2 * (lane & 1) + ((lane >> 1) & 1);
       if (lane < 4 && e < S) slot[size_t(e) * a.strips] = 0.0625f * k;
