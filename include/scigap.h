@@ -315,8 +315,9 @@ typedef struct scigap_unrolled {
 size_t scigap_unrolled_checkpoint_bytes(const scigap_unrolled* u);
 
 /* Workspace of a forward or a backward call (the same size for both);
- * with batch > 1 it holds the scratch of up to 4 samples, which run
- * together (one launch per step for all of them). */
+ * with batch > 1 it holds the scratch of a group of samples, which run
+ * together (one launch per step for all of them): up to 4, up to 8 with
+ * tv_iter_max 6 and 7. */
 size_t scigap_unrolled_workspace_bytes(const scigap_unrolled* u);
 
 /* Forward: x_out (batch,T,H,W) = x_K of every sample.  lambdas and weights

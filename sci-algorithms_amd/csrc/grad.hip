@@ -39,7 +39,8 @@ namespace scigap {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kSamples = 4;  // samples of one launch (a group)
+constexpr int kSamples = 4;   // samples of one launch (a group), as a rule
+constexpr int kSamplesMax = 8;
 
 // Block reduction of one float into a gradient accumulator's slot.
 __device__ __forceinline__ void block_atomic(float v, double* dst) {
@@ -358,6 +359,7 @@ bool proj_vector(int64_t N, std::initializer_list<const void*> ptrs,
 
 }  // namespace
 
+int64_t tv_backward_rounds(int D, int nb, int64_t H, int64_t W, int64_t T);
 int tv_backward_tiles(int D, int nb, const float* x, size_t x_b, const float* phi, const float* r,
                       size_t r_b, float lam, const float* xbar, size_t xbar_b, const float* ybb,
                       size_t ybb_b, float* vbar, size_t vbar_b, int64_t H, int64_t W, int64_t T,
@@ -504,8 +506,8 @@ CkptLayout ckpt_layout(const scigap_unrolled& u) {
   return c;
 }
 
-// Workspace: the samples of a batch run in groups of up to kSamples, one
-// launch per step for the whole group.
+// Workspace: the samples of a batch run in groups (group_of), one launch per
+// step for the whole group.
 struct UWorkspace {
   float* phi = nullptr;      // sigmoid(logits), when logits
   float* S = nullptr;        // phi_sum
@@ -520,7 +522,29 @@ struct UWorkspace {
   size_t bytes = 0;
 };
 
-int group_of(const scigap_unrolled& u) { return u.batch < kSamples ? u.batch : kSamples; }
+// Samples of a group: four fill the GPU and bound the scratch.  The reverse TV
+// of 5 and 6 updates has one large workgroup per tile and CU, and a group waits
+// for its last, partly empty round of them: there the size up to eight with the
+// fewest rounds, a group's other launches counted as one round (36 us).  144
+// workgroups a sample at 256x256x8, 6 updates: a batch of 8 takes 5 rounds, as
+// 4 + 4 six; of 6 four, as 4 + 2 five.
+int group_of(const scigap_unrolled& u) {
+  const int D = u.tv_iter_max - 1;
+  int best = u.batch < kSamples ? u.batch : kSamples;
+  if (D <= 4) return best;
+  auto cost = [&](int g) {
+    const int64_t full = u.batch / g, rest = u.batch % g;
+    return full * (tv_backward_rounds(D, g, u.H, u.W, u.T) + 1) +
+           (rest ? tv_backward_rounds(D, int(rest), u.H, u.W, u.T) + 1 : 0);
+  };
+  int64_t least = cost(best);
+  for (int g = 1; g <= u.batch && g <= kSamplesMax; ++g)
+    if (cost(g) < least) {
+      least = cost(g);
+      best = g;
+    }
+  return best;
+}
 
 UWorkspace carve(const scigap_unrolled& u, char* base) {
   const size_t N = size_t(u.H) * u.W, V = N * size_t(u.T), K = size_t(u.iters);
@@ -630,8 +654,9 @@ int scigap_unrolled_forward(const scigap_unrolled* u, const float* lambdas, cons
   const float* phi = nullptr;
   if (int rc = prepare_mask(*u, mask, w, &phi, s)) return rc;
   const size_t dist = cl.per_sample / 4;  // distance between samples in floats
-  for (int b = 0; b < u->batch; b += kSamples) {
-    const int nb = u->batch - b < kSamples ? u->batch - b : kSamples;
+  const int group = group_of(*u);
+  for (int b = 0; b < u->batch; b += group) {
+    const int nb = u->batch - b < group ? u->batch - b : group;
     char* cb = static_cast<char*>(ckpt) + cl.per_sample * b;
     float* xs = reinterpret_cast<float*>(cb + cl.x);
     float* rs = reinterpret_cast<float*>(cb + cl.r);
@@ -677,8 +702,8 @@ int scigap_unrolled_backward(const scigap_unrolled* u, const float* lambdas, con
   const size_t dist = cl.per_sample / 4;
   const int group = group_of(*u);
   float* const phibar = grad_mask ? w.phibar : nullptr;
-  for (int b = 0; b < u->batch; b += kSamples) {
-    const int nb = u->batch - b < kSamples ? u->batch - b : kSamples;
+  for (int b = 0; b < u->batch; b += group) {
+    const int nb = u->batch - b < group ? u->batch - b : group;
     const char* cb = static_cast<const char*>(ckpt) + cl.per_sample * b;
     const GroupCkpt c{reinterpret_cast<const float*>(cb + cl.x), cl.xstride, dist,
                       reinterpret_cast<const float*>(cb + cl.r), cl.rstride, dist,

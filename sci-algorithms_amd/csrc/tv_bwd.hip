@@ -389,10 +389,15 @@ __global__ void __launch_bounds__(64 * kBwdBY) k_tv_bwd(BwdArgs a) {
 }
 
 template <int D>
-int launch_tv_bwd(BwdArgs a, int T, hipStream_t s) {
+void set_bwd_tiles(BwdArgs& a) {
   using G = BwdGeom<D>;
   a.tiles_x = tiles_across(a.W, G::LW, G::HC, G::OX);
   a.tiles_y = tiles_across(a.H, G::LH, G::HR, G::OY);
+}
+
+template <int D>
+int launch_tv_bwd(BwdArgs a, int T, hipStream_t s) {
+  set_bwd_tiles<D>(a);
   k_tv_bwd<D><<<dim3(unsigned(a.tiles_x * a.tiles_y), unsigned(T), unsigned(a.nb)), 64 * kBwdBY, 0,
                 s>>>(a);
   SCIGAP_LAUNCH_CHECK("fused TV backward launch");
@@ -677,6 +682,21 @@ int launch_tv_bwd_sweep(const BwdArgs& a, int T, hipStream_t s) {
 }
 
 }  // namespace
+
+// Rounds of workgroups (one per CU at a time) that the reverse TV of nb samples
+// takes; 0 for the row sweeps, whose waves are many and small.
+int64_t tv_backward_rounds(int D, int nb, int64_t H, int64_t W, int64_t T) {
+  if (D <= 4) return 0;
+  BwdArgs a{};
+  a.H = int(H);
+  a.W = int(W);
+  if (D == 5)
+    set_bwd_tiles<5>(a);
+  else
+    set_bwd_tiles<6>(a);
+  const int64_t cus = std::max(device_simds() / 4, 1);
+  return (int64_t(a.tiles_x) * a.tiles_y * T * nb + cus - 1) / cus;
+}
 
 // vbar = (d out_D / d v)^T xbar for every frame, and wbar += xbar . d out_D / dw,
 // for D fixed Chambolle updates with weight w on v = x + (lam r) Phi (D in
