@@ -1,4 +1,5 @@
-// Row-sweep engine of the Chambolle TV for gfx950 (device code only).
+// Row-sweep engine of the Chambolle TV for gfx950: the device code of a strip, and
+// how an image is cut into strips.
 //
 // One wavefront carries a 128-column strip of one frame down its rows with all
 // S dual updates in flight at once, each one row behind the one before it:
@@ -20,6 +21,8 @@
 // strips are placed by the same col_place.
 #pragma once
 
+#include <algorithm>
+#include <cmath>
 #include <utility>
 
 #include "fused.h"
@@ -43,6 +46,46 @@ extern "C" __device__ void raw_buffer_store_f2(f2 v, __amdgpu_buffer_rsrc_t rsrc
 __device__ __forceinline__ float uniform(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
+
+// ---------------------------------------------------------------------------
+// Passes and strips of the deep TV (host)
+// ---------------------------------------------------------------------------
+
+constexpr int kMaxPass = 6;  // updates of a pass
+
+// Strips up to which every wave sums its frame's energy slots itself: 6 slot
+// rows of 128 are 12 loads a lane, about the launch they replace (512x512x10,
+// 29 updates: 152 us with a limit of 64 or 128, 162 us with 300).
+constexpr int kInlineStrips = 128;
+
+// Strips across an image for passes of S updates (column halo HC(S)).
+inline int strips_across(int W, int S) {
+  const int HC = (S + 2) & ~1;
+  return tiles_across(W, 128, HC, 128 - 2 * HC);
+}
+
+// Rows a strip owns: tall strips waste fewer halo rows, short ones give more
+// waves.  The sweep of one strip costs S*(R + S) row updates; a SIMD works its
+// waves off one after the other, and is about 2/3 busy with a single one.
+// (29 updates, R = 8 / 16 / 32 / 64: 75 / 94 / 139 / - us at 256x256x8, 330 /
+// 297 / 308 / - us at 1024x1024x8, 2.65 / 2.17 / 1.97 / 2.02 ms at
+// 2048x2048x20.)
+inline int strip_rows(int64_t H, int64_t W, int64_t T, int S, int simds) {
+  int best = 8;
+  double best_cost = 1e300;
+  for (int R : {8, 16, 32, 64}) {
+    const double waves = double(strips_across(int(W), S)) * double((H + R - 1) / R) * double(T);
+    const double per_simd = std::max(1.5, std::ceil(waves / simds));
+    const double cost = per_simd * double(R + S + 3);
+    if (cost < best_cost * 0.999) {
+      best_cost = cost;
+      best = R;
+    }
+  }
+  return best;
+}
+
+// ---------------------------------------------------------------------------
 
 // Where a strip's pixels are.
 struct StripPos {

@@ -38,14 +38,8 @@ namespace {
 
 using namespace sweep;
 
-constexpr int kMaxPass = 6;
 constexpr int kWaves = 4;   // independent waves of one workgroup
 constexpr int kAheadTv = 2; // rows requested ahead of their use (4: no faster)
-
-// Strips up to which every wave sums its frame's energy slots itself: 6 slot
-// rows of 128 are 12 loads a lane, about the launch they replace (512x512x10,
-// 29 updates: 152 us with a limit of 64 or 128, 162 us with 300).
-constexpr int kInlineStrips = 128;
 
 struct PassArgs {
   const float* img;    // (T,H,W)
@@ -250,33 +244,6 @@ __global__ void __launch_bounds__(64 * kMaxPass) k_tv_decide(PassArgs a) {
   }
 }
 
-// Strips across an image for passes of S updates (column halo HC(S)).
-int strips_across(int W, int S) {
-  const int HC = (S + 2) & ~1;
-  return tiles_across(W, 128, HC, 128 - 2 * HC);
-}
-
-// Rows a strip owns: tall strips waste fewer halo rows, short ones give more
-// waves.  The sweep of one strip costs S*(R + S) row updates; a SIMD works its
-// waves off one after the other, and is about 2/3 busy with a single one.
-// (29 updates, R = 8 / 16 / 32 / 64: 75 / 94 / 139 / - us at 256x256x8, 330 /
-// 297 / 308 / - us at 1024x1024x8, 2.65 / 2.17 / 1.97 / 2.02 ms at
-// 2048x2048x20.)
-int pick_rows(int64_t H, int64_t W, int64_t T, int S, int simds) {
-  int best = 8;
-  double best_cost = 1e300;
-  for (int R : {8, 16, 32, 64}) {
-    const double waves = double(strips_across(int(W), S)) * double((H + R - 1) / R) * double(T);
-    const double per_simd = std::max(1.5, std::ceil(waves / simds));
-    const double cost = per_simd * double(R + S + 3);
-    if (cost < best_cost * 0.999) {
-      best_cost = cost;
-      best = R;
-    }
-  }
-  return best;
-}
-
 template <int S>
 void launch_pass(const PassArgs& a, int pass, hipStream_t s) {
   const unsigned grid = unsigned(a.per_xcd * 8);
@@ -350,7 +317,7 @@ int tv_sweep(const float* image, float* out, int64_t H, int64_t W, int64_t T, fl
   a.weight = weight;
   a.tw = float(0.25 / double(weight));
   a.eps = eps;
-  a.R = pick_rows(H, W, T, low, device_simds());
+  a.R = strip_rows(H, W, T, low, device_simds());
   int i0 = 0;
   for (int c = 0; c <= passes; ++c) {
     const bool finish = c == passes;
