@@ -460,8 +460,9 @@ __device__ __forceinline__ void fused_strip(const FusedArgs& a, int tile,
       }
     }
   }
-  // (after the first loads' requests: before them, a workgroup with one frame
-  // held its memory latency that much longer, 2% of the launch at 1500x1500x1)
+  // (After the first loads' requests: before them, a workgroup with one frame
+  // held its memory latency that much longer.  An iteration of 1500x1500x1 with 2
+  // dual updates 33.0 us, now 32.0; of 801x1003x2 with 4 26.1, now 25.7.)
   zero_energies<D, BY, ENERGY>(red);
   float err = 0.f;
 
@@ -823,8 +824,9 @@ __host__ __device__ inline bool tile_inside(int tile, int tiles_x, int H, int W)
 }
 
 // One launch covers interior and border tiles.  PART restricts a launch to
-// one class (1: interior, 2: border; 0: both), so that the interior kernel is
-// allocated registers for its own body only.  MANY: several solves share the
+// one class (1: interior, 2: border; 0: both); its strips are masked one by one
+// as well, which is up to 4% faster than one body per launch for 8-row tiles and
+// up to 4% slower for 16-row ones.  MANY: several solves share the
 // launch; a kernel of its own, because the arguments of a solve chosen at run
 // time take scalar registers that every strip body is short of (one kernel for
 // both: 66 of them spilled instead of 55 in GAP, 1-2% of the launch for sizes
