@@ -193,6 +193,8 @@ def sq_error(a, b, per_frame: bool = False):
     """sum((a-b)^2) in fp64 over (T,H,W) tensors (per frame if requested)."""
     torch = _torch()
     T, H, W = a.shape
+    if b.numel() < a.numel():  # would be read past its end
+        raise ValueError("shapes differ: %s and %s" % (tuple(a.shape), tuple(b.shape)))
     out = torch.empty(T if per_frame else 1, dtype=torch.float64, device=a.device)
     L = _lib.lib()
     _lib.check(L.scigap_sq_error(a.data_ptr(), b.data_ptr(), out.data_ptr(), H, W, T,

@@ -32,6 +32,8 @@ def ssim_frames(truth, x, data_range: float = 1.0):
     T, H, W = x.shape
     if min(H, W) < 7:
         raise ValueError("win_size exceeds image extent.  If the input is a multichannel (color) image, set multichannel=True.")
+    if truth.numel() < x.numel():  # would be read past its end
+        raise ValueError("shapes differ: %s and %s" % (tuple(truth.shape), tuple(x.shape)))
     out = torch.empty(T, dtype=torch.float64, device=x.device)
     L = _lib.lib()
     _lib.check(L.scigap_ssim(truth.data_ptr(), x.data_ptr(), out.data_ptr(), H, W, T,

@@ -109,6 +109,11 @@ def solve_device(y, phi, phi_sum, *, method="gap", iters=50, _lambda=1.0, accele
                 raise ValueError("solves that share launches need contiguous tensors with one "
                                  "leading dimension: got %s, expected %s"
                                  % (tuple(v.shape), lead + want))
+    for name, v, n in (("y", y, H * W), ("phi_sum", phi_sum, H * W), ("x0", x0, T * H * W),
+                       ("truth", truth, T * H * W)):
+        if v is not None and v.numel() < n:  # would be read past its end
+            raise ValueError("%s has %d elements, a %dx%dx%d solve reads %d"
+                             % (name, v.numel(), H, W, T, n))
     p = _lib.Params()
     L = _lib.lib()
     L.scigap_default_params(p, H, W, T)

@@ -32,3 +32,14 @@ def test_subgrids_in_turn_match_shared_launches(gpu, monkeypatch, H, W, T, warm,
     assert len(p) == len(pt) == len(s) == len(st) == (T if iqa else 0)
     assert np.allclose(p, pt, atol=1e-2) and np.allclose(s, st, atol=1e-4)
     assert len(pa) == len(pat) == (6 if iqa else 0) and np.allclose(pa, pat, atol=1e-2)
+
+
+def test_short_warm_start_or_truth_is_refused(gpu, monkeypatch):
+    import pnp_sci
+    from pnp_sci import pnp_sci_algo as algo
+    mask = np.ones((16, 20, 3), np.float32)
+    for voxels in (algo._SHARED_SOLVE_VOXELS, 0):
+        monkeypatch.setattr(algo, "_SHARED_SOLVE_VOXELS", voxels)
+        for short in (dict(x0_bayer=mask[..., :2]), dict(X_orig=mask[..., :2])):
+            with pytest.raises(ValueError):
+                pnp_sci.gap_denoise_bayer(mask.sum(2), mask, iter_max=2, **short)
