@@ -228,7 +228,7 @@ struct Rows {
   int lim = S;    // LIMIT only; wave-uniform
   // 16 times this lane's part of E_u over the owned rows: `acc` adds up kSumRows
   // rows, `tot` those sums, so that no chain of fp32 additions grows with the
-  // strip's height (64 rows: 256 terms in one, up to 3e-6 of their sum).
+  // strip's height (all terms of 64 rows in one chain: 1.9e-6 of the sum of a ramp).
   static constexpr int kSumRows = 4;
   float acc[S] = {}, tot[S] = {};
 
